@@ -102,6 +102,10 @@ bool launch_xbwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_zbwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 bool launch_zfwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
+// two-pass FFTs of runtime factors; return false for lengths without a factor pair of the list
+bool launch_xprod_line(const XArgs &a, bool fp32, hipStream_t st);
+bool launch_zbwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);
+bool launch_zfwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 
 // ----------------------------------------------------------- spectral ----
 struct LayoutArgs {

@@ -9,6 +9,8 @@
 //   x stage : c2r of (u,v,w,wx,wy,wz) packed two real lines per complex FFT, the cross
 //             product in LDS, and r2c of the three products, in one kernel, so that the
 //             nine physical fields never reach HBM.
+// The FFT kernels of this file serve the lengths that neither transforms_rf.hip (tuned) nor
+// transforms_line.hip (factor pairs up to 27) takes, e.g. 245 = 5 x 49, and CDNS_FFT=stockham.
 // Normalisation follows transforms.cpp exactly: backward synthesis is the exact value of
 // the truncated series; forward applies 1/NX2 (no Nyquist halving), 1/NZ2 and the DCT-I
 // weights 1/(2 NY2) (iy=0), 1/NY2 (iy>=1).
@@ -448,7 +450,7 @@ static int items_per_thread(int nlines, const FftPlan &p) {
 }
 
 void launch_zbwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st) {
-    if (a.rf && launch_zbwd_rf(a, nfields, fp32, st)) return;
+    if (a.rf && (launch_zbwd_rf(a, nfields, fp32, st) || launch_zbwd_line(a, nfields, fp32, st))) return;
     const int it = items_per_thread(a.KT, a.plan);
     dim3 grid((a.nkx + a.KT - 1) / a.KT, a.NL, nfields);
     if (fp32) {
@@ -460,7 +462,7 @@ void launch_zbwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st) {
     }
 }
 void launch_zfwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st) {
-    if (a.rf && launch_zfwd_rf(a, nfields, fp32, st)) return;
+    if (a.rf && (launch_zfwd_rf(a, nfields, fp32, st) || launch_zfwd_line(a, nfields, fp32, st))) return;
     const int it = items_per_thread(a.KT, a.plan);
     dim3 grid((a.nkx + a.KT - 1) / a.KT, a.NL, nfields);
     if (fp32) {
@@ -472,7 +474,7 @@ void launch_zfwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st) {
     }
 }
 void launch_xprod(const XArgs &a, bool fp32, hipStream_t st) {
-    if (a.rf && launch_xprod_rf(a, fp32, st)) return;
+    if (a.rf && (launch_xprod_rf(a, fp32, st) || launch_xprod_line(a, fp32, st))) return;
     const int it = items_per_thread(3 * a.P, a.plan);
     if ((a.P / 2) * a.plan.n > 8 * 256) throw std::runtime_error("x-product batch too large");
     dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P);
