@@ -89,28 +89,58 @@ void launch_wall_sum(const zd *nly, const zd *bcw, zd *pbc, int ny, int JS, int 
     else hipLaunchKernelGGL((k_wall_sum<2>), grid, block, 0, st, nly, bcw, pbc, ny, JS, NQ);
 }
 
-// reference (izi, row, kx, c) -> plane c, column q = kx*nzk + izi, row (padding rows zeroed)
-__global__ void k_ref_to_planes(LayoutArgs a) {
-    const size_t total = (size_t)a.nkx * a.nzk * a.JS;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-        const int row = (int)(e % a.JS);
-        const size_t q = e / a.JS;
-        const int kx = (int)(q / a.nzk), izi = (int)(q % a.nzk);
-        for (int c = 0; c < a.ncomp; ++c) {
-            zd v = {0.0, 0.0};
-            if (row < a.nrow) v = a.ref_in[(((size_t)izi * a.nrow + row) * a.nkx + kx) * a.stride + c];
-            a.plane_out[c][e] = v;
-        }
+// Reference layout (izi, row, kx, c) <-> plane c, column q = kx*nzk + izi, row.  For one izi this is a
+// transpose of (row, kx) per component: a block carries a tile of kLayRows rows x TK kx through LDS, so
+// that the reference side moves runs of TK*NC values (768 bytes for vectors) and the plane side runs of
+// kLayRows values (512 bytes).  HBM-bound; without the tile one side moved single 16-byte values at a
+// stride of a row (Re_tau=180: velocity to planes 45.8 -> 23.9 us with it, velocity and pressure back
+// 64 -> 33 us; 102 MB and 136 MB).
+constexpr int kLayRows = 32;
+template <int NC> constexpr int kLayKx = NC == 1 ? 32 : 16;
+template <int NC> struct LayTile {
+    static constexpr int TK = kLayKx<NC>, W = TK * NC, PITCH = kLayRows + 1, N = kLayRows * W;
+    // entry of component c, tile column k, tile row r
+    __device__ static inline int at(int c, int k, int r) { return (c * TK + k) * PITCH + r; }
+};
+
+// rows beyond nrow (the planes' padding) are written as zeros
+template <int NC> __global__ void __launch_bounds__(256) k_ref_to_planes(LayoutArgs a) {
+    using T = LayTile<NC>;
+    __shared__ zd tile[NC * T::TK * T::PITCH];
+    const int kx0 = blockIdx.x * T::TK, r0 = blockIdx.y * kLayRows, izi = blockIdx.z;
+    const zd *ref = a.ref_in + (size_t)izi * a.nrow * a.nkx * a.stride;
+#pragma unroll
+    for (int e = threadIdx.x; e < T::N; e += 256) {
+        const int r = e / T::W, w = e - r * T::W, k = w / NC, c = w - k * NC;
+        const bool in = r0 + r < a.nrow && kx0 + k < a.nkx;
+        const zd v = ref[in ? ((size_t)(r0 + r) * a.nkx + kx0 + k) * a.stride + c : 0];
+        tile[T::at(c, k, r)] = in ? v : zd{0.0, 0.0};
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = threadIdx.x; e < T::N; e += 256) {
+        const int w = e / kLayRows, r = e - w * kLayRows, c = w / T::TK, k = w - c * T::TK;
+        if (r0 + r < a.JS && kx0 + k < a.nkx)
+            a.plane_out[c][((size_t)(kx0 + k) * a.nzk + izi) * a.JS + r0 + r] = tile[T::at(c, k, r)];
     }
 }
-__global__ void k_planes_to_ref(LayoutArgs a) {
-    const size_t total = (size_t)a.nzk * a.nrow * a.nkx;
-    for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-        const int kx = (int)(e % a.nkx);
-        const size_t r = e / a.nkx;
-        const int row = (int)(r % a.nrow), izi = (int)(r / a.nrow);
-        const size_t src = ((size_t)kx * a.nzk + izi) * a.JS + row;
-        for (int c = 0; c < a.ncomp; ++c) a.ref_out[e * a.stride + c] = a.plane_in[c][src];
+template <int NC> __global__ void __launch_bounds__(256) k_planes_to_ref(LayoutArgs a) {
+    using T = LayTile<NC>;
+    __shared__ zd tile[NC * T::TK * T::PITCH];
+    const int kx0 = blockIdx.x * T::TK, r0 = blockIdx.y * kLayRows, izi = blockIdx.z;
+#pragma unroll
+    for (int e = threadIdx.x; e < T::N; e += 256) {
+        const int w = e / kLayRows, r = e - w * kLayRows, c = w / T::TK, k = w - c * T::TK;
+        const bool in = r0 + r < a.nrow && kx0 + k < a.nkx;
+        tile[T::at(c, k, r)] = a.plane_in[c][in ? ((size_t)(kx0 + k) * a.nzk + izi) * a.JS + r0 + r : 0];
+    }
+    __syncthreads();
+    zd *ref = a.ref_out + (size_t)izi * a.nrow * a.nkx * a.stride;
+#pragma unroll
+    for (int e = threadIdx.x; e < T::N; e += 256) {
+        const int r = e / T::W, w = e - r * T::W, k = w / NC, c = w - k * NC;
+        if (r0 + r < a.nrow && kx0 + k < a.nkx)
+            ref[((size_t)(r0 + r) * a.nkx + kx0 + k) * a.stride + c] = tile[T::at(c, k, r)];
     }
 }
 __global__ void k_real_planes_to_ref(const double *plane, double *ref, int nrow, int nkx, int nzk, int JS) {
@@ -144,11 +174,18 @@ void launch_widen(const void *src, zd *dst, size_t n, hipStream_t st) {
 void launch_narrow(const zd *src, void *dst, size_t n, hipStream_t st) {
     hipLaunchKernelGGL(k_narrow, grid_for(n), dim3(256), 0, st, src, reinterpret_cast<cpx<float> *>(dst), n);
 }
+template <int NC> static dim3 layout_grid(const LayoutArgs &a, int rows) {
+    return dim3((a.nkx + kLayKx<NC> - 1) / kLayKx<NC>, (rows + kLayRows - 1) / kLayRows, a.nzk);
+}
 void launch_ref_to_planes(const LayoutArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL(k_ref_to_planes, grid_for((size_t)a.nkx * a.nzk * a.JS), dim3(256), 0, st, a);
+    if (a.ncomp == 1) hipLaunchKernelGGL(k_ref_to_planes<1>, layout_grid<1>(a, a.JS), dim3(256), 0, st, a);
+    else if (a.ncomp == 3) hipLaunchKernelGGL(k_ref_to_planes<3>, layout_grid<3>(a, a.JS), dim3(256), 0, st, a);
+    else throw std::runtime_error("unsupported number of components");
 }
 void launch_planes_to_ref(const LayoutArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL(k_planes_to_ref, grid_for((size_t)a.nzk * a.nrow * a.nkx), dim3(256), 0, st, a);
+    if (a.ncomp == 1) hipLaunchKernelGGL(k_planes_to_ref<1>, layout_grid<1>(a, a.nrow), dim3(256), 0, st, a);
+    else if (a.ncomp == 3) hipLaunchKernelGGL(k_planes_to_ref<3>, layout_grid<3>(a, a.nrow), dim3(256), 0, st, a);
+    else throw std::runtime_error("unsupported number of components");
 }
 void launch_real_planes_to_ref(const double *plane, double *ref, int nrow, int nkx, int nzk, int JS, hipStream_t st) {
     hipLaunchKernelGGL(k_real_planes_to_ref, grid_for((size_t)nzk * nrow * nkx), dim3(256), 0, st, plane, ref, nrow,
