@@ -82,11 +82,13 @@ constexpr int kYCurlWaves = 4;
 constexpr int kYCurlLds = 64 * 1024;
 // forward: waves per block (the parts' tables are shared by all of a block's column groups)
 constexpr int kYFwdWaves = 8;
+// waves per block of the y stages of small grids
+constexpr int kYSmallWaves = 4;
 
 // ------------------------------------------------------------------ backward --
-// grid: (column groups of 8 waves, row parts, fields); TRP row tiles (16 l' each) per part.
-template <typename R, int TRP, int CT>
-__global__ void __launch_bounds__(64 * kWaves) k_ybwd_mfma(YArgs a) {
+// grid: (column groups of W waves, row parts, fields); TRP row tiles (16 l' each) per part.
+template <typename R, int TRP, int CT, int W>
+__global__ void __launch_bounds__(64 * W) k_ybwd_mfma(YArgs a) {
     using M = Mfma<R>;
     using v4 = typename M::v4;
     constexpr int PITCH = TRP * 16;
@@ -114,7 +116,7 @@ __global__ void __launch_bounds__(64 * kWaves) k_ybwd_mfma(YArgs a) {
 
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int col = lane & 15, k = lane >> 4, hh = col & 1;
-    const int qb = (cg * kWaves + wv) * 8 * CT;
+    const int qb = (cg * W + wv) * 8 * CT;
     // FP32: lane (col, k) loads the whole complex S[q][8s + 2k + (col & 1)], q = qb + 8c + col/2,
     // so that each load instruction reads eight columns x 128 contiguous bytes; the MFMA operands
     // are one part of the even-j and one of the odd-j value, its own and its pair partner's (DPP
@@ -676,12 +678,11 @@ __global__ void __launch_bounds__(64 * W) k_yfwd_mfma(YArgs a) {
 
 // --------------------------------------------------------------------- launch --
 // 1-D grids of (parts x column groups x fields) blocks, decoded by xcd_block.
-template <typename R, int TRP, int CT> static void go_ybwd(YArgs a, int parts, int nf, hipStream_t st) {
+template <typename R, int TRP, int W> static void go_ybwd(YArgs a, int parts, int nf, hipStream_t st) {
     const size_t sm = ((size_t)a.njp * TRP * 16 + a.njp) * sizeof(R);
-    const int cols = 8 * CT * kWaves;
     a.parts = parts;
-    a.ncg = (a.NQ + cols - 1) / cols;
-    hipLaunchKernelGGL((k_ybwd_mfma<R, TRP, CT>), dim3(a.parts * a.ncg * nf, 1), dim3(64 * kWaves), sm, st, a);
+    a.ncg = (a.NQ + 8 * W - 1) / (8 * W);
+    hipLaunchKernelGGL((k_ybwd_mfma<R, TRP, 1, W>), dim3(a.parts * a.ncg * nf, 1), dim3(64 * W), sm, st, a);
 }
 template <typename R, int JTP, int CT, int W = kYFwdWaves>
 static void go_yfwd(YArgs a, int parts, int nf, hipStream_t st) {
@@ -708,28 +709,37 @@ static int tiles_per_part(size_t bytes_per_tile, size_t fixed, int cap) {
     return t;
 }
 
+// compute units of the device current at the first call (256 if the query fails); the static's
+// initialisation runs once, also when several host threads launch
+static int device_cus() {
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) == hipSuccess &&
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
+            return n;
+        return 256;
+    }();
+    return cus;
+}
+
 bool launch_ybwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     y_shape(a);
     const size_t esz = fp32 ? 4 : 8;
     const int TR = (a.rows_m + 15) / 16;
     if ((size_t)a.njp * 16 * esz + a.njp * esz > (size_t)kLdsBudget) return false;
-    const int fit = std::min(tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, 4), TR);
-    const int parts = (TR + fit - 1) / fit;
-    const int trp = (TR + parts - 1) / parts; // balanced parts; the kernel masks rows >= rows_m
+    // Two row tiles per wavefront on 8-wavefront blocks; where that grid has fewer blocks than the
+    // device CUs, one row tile on 4-wavefront blocks (four times the blocks, half the work of each).
+    // us per launch, FP64, two tiles / one tile (the three tiles per part that filled the LDS before):
+    // 196 x 193 x 196 1 field 18.6 / 22.8 (25.2), 6 fields 81.7 / 109.8 (84.1); 96 x 97 x 96 1 field
+    // 9.7 / 7.8 (11.7), 6 fields 15.5 / 15.3 (15.8); 150 x 136 x 126, 204 blocks, 1 field 11.7 / 11.4 (14.7).
+    const int ncg = (a.NQ + 8 * kWaves - 1) / (8 * kWaves), trp = tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, 2);
+    const bool small = trp == 1 || ncg * ((TR + 1) / 2) * nf < device_cus();
     if (fp32) {
-        switch (trp) {
-        case 1: go_ybwd<float, 1, 1>(a, parts, nf, st); break;
-        case 2: go_ybwd<float, 2, 1>(a, parts, nf, st); break;
-        case 3: go_ybwd<float, 3, 1>(a, parts, nf, st); break;
-        default: go_ybwd<float, 4, 1>(a, parts, nf, st); break;
-        }
+        if (small) go_ybwd<float, 1, kYSmallWaves>(a, TR, nf, st);
+        else go_ybwd<float, 2, kWaves>(a, (TR + 1) / 2, nf, st);
     } else {
-        switch (trp) {
-        case 1: go_ybwd<double, 1, 1>(a, parts, nf, st); break;
-        case 2: go_ybwd<double, 2, 1>(a, parts, nf, st); break;
-        case 3: go_ybwd<double, 3, 1>(a, parts, nf, st); break;
-        default: go_ybwd<double, 4, 1>(a, parts, nf, st); break;
-        }
+        if (small) go_ybwd<double, 1, kYSmallWaves>(a, TR, nf, st);
+        else go_ybwd<double, 2, kWaves>(a, (TR + 1) / 2, nf, st);
     }
     return true;
 }
@@ -765,19 +775,6 @@ bool launch_ybwd_curl(YArgs a, bool fp32, hipStream_t st) {
     return true;
 }
 
-// compute units of the device current at the first call (256 if the query fails); the static's
-// initialisation runs once, also when several host threads launch
-static int device_cus() {
-    static const int cus = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-            return n;
-        return 256;
-    }();
-    return cus;
-}
-
 bool launch_yfwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     y_shape(a);
     const size_t esz = fp32 ? 4 : 8;
@@ -786,17 +783,15 @@ bool launch_yfwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     const int fit = std::min(tiles_per_part((size_t)2 * a.KL * 16 * esz + 16 * esz, 0, 2), JT);
     const int parts = (JT + fit - 1) / fit;
     const int jtp = (JT + parts - 1) / parts;
-    // a grid of fewer 8-wavefront blocks of two column sets than the device has CUs (small meshes:
-    // 51 blocks at 64x65x64) runs one column set per wavefront in 2-wavefront blocks, eight times
-    // the blocks; each column's matrix operations are the same either way
+    // a grid of fewer 8-wavefront blocks of two column sets than the device has CUs (small meshes, single
+    // fields) runs one column set and one j tile per wavefront in 4-wavefront blocks: up to eight times the
+    // blocks, and half the table in each block's LDS; each column's matrix operations are the same either
+    // way.  us per launch, FP64, against two column sets / the 2-wavefront blocks with whole tables that
+    // small grids had before: 96 x 97 x 96 3 fields 10.5 (16.6 / 13.1), 150 x 136 x 126 3 fields (204 blocks)
+    // 20.4 (23.1 / 40.6), 196 x 193 x 196 1 field (132 blocks) 20.1 (23.7 / 31.7), 3 fields (396 blocks) 42.8 (39.1 / 72.7)
     if (parts * ((a.NQ + 8 * 2 * kYFwdWaves - 1) / (8 * 2 * kYFwdWaves)) * nf < device_cus()) {
-        if (fp32) {
-            if (jtp == 1) go_yfwd<float, 1, 1, 2>(a, parts, nf, st);
-            else go_yfwd<float, 2, 1, 2>(a, parts, nf, st);
-        } else {
-            if (jtp == 1) go_yfwd<double, 1, 1, 2>(a, parts, nf, st);
-            else go_yfwd<double, 2, 1, 2>(a, parts, nf, st);
-        }
+        if (fp32) go_yfwd<float, 1, 1, kYSmallWaves>(a, JT, nf, st);
+        else go_yfwd<double, 1, 1, kYSmallWaves>(a, JT, nf, st);
         return true;
     }
     if (fp32) {
