@@ -525,7 +525,7 @@ void coarse_backward(cdns_ctx *c, const zd *plane, double *phys) {
     }
     {
         Launch L(c, "coarse_x_backward");
-        launch_xbwd_phys(xargs_coarse(c, c->Zbuf, nullptr, phys), false, c->st);
+        launch_xbwd_phys(xargs_coarse(c, c->Zbuf, nullptr, phys), 1, false, c->st);
     }
 }
 // coarse physical field (device) -> spectral plane
@@ -1467,7 +1467,7 @@ int cdns_xyzfft2(cdns_ctx *c, char dir, double *phys, double *spec, int stride, 
             a.phys = dphys;
             {
                 Launch L(c, "x_backward");
-                launch_xbwd_phys(a, c->fp32, c->st);
+                launch_xbwd_phys(a, 1, c->fp32, c->st);
             }
             if (where == CDNS_HOST) {
                 CDNS_HIP(hipMemcpyAsync(phys, dphys, np * sizeof(double), hipMemcpyDeviceToHost, c->st));

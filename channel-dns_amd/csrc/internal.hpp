@@ -78,7 +78,8 @@ struct XArgs {
     int rf;
     int pair; // product: rows of the register FFT on lane pairs (even factors)
     int coarse; // coarse-grid transform: at NXS = N/2 the Nyquist coefficient counts twice
-    double *phys; // reference-layout physical field for the single-field stages
+    double *phys; // reference-layout physical field(s) for the single-field stages
+    size_t phys_fs; // x backward of several fields: stride of the physical fields
     // product a x b: input fields a0 a1 a2 b0 b1 b2 and the three output fields
     const void *fin[6];
     void *fout[3];
@@ -93,17 +94,17 @@ void launch_yfwd(const YArgs &a, int nfields, bool fp32, hipStream_t st);
 void launch_zbwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st);
 void launch_zfwd(const ZArgs &a, int nfields, bool fp32, hipStream_t st);
 void launch_xprod(const XArgs &a, bool fp32, hipStream_t st);
-void launch_xbwd_phys(const XArgs &a, bool fp32, hipStream_t st);
+void launch_xbwd_phys(const XArgs &a, int nfields, bool fp32, hipStream_t st);
 void launch_xfwd_phys(const XArgs &a, bool fp32, hipStream_t st);
 // register-resident two-pass FFT variants; return false for lengths without an instantiation
 bool rf_supported(int n);
 bool launch_xprod_rf(const XArgs &a, bool fp32, hipStream_t st);
-bool launch_xbwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st);
-bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_zbwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 bool launch_zfwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 // two-pass FFTs of runtime factors; return false for lengths without a factor pair of the list
 bool launch_xprod_line(const XArgs &a, bool fp32, hipStream_t st);
+bool launch_xbwd_phys_line(const XArgs &a, int nf, bool fp32, hipStream_t st);
+bool launch_xfwd_phys_line(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_zbwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 bool launch_zfwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 

@@ -273,92 +273,6 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
     }
 }
 
-// ------------------------------------------- single-field x stages (physical) --
-// Two points share one complex line: a + i b.
-template <typename R, int N1, int N2>
-__global__ void __launch_bounds__(64) k_xbwd_phys_rf(XArgs a) {
-    using Gm = Geo<N1, N2>;
-    constexpr int N = Gm::N, MX = Gm::MX, G = Gm::G, NG = Gm::NG, LB = Gm::LB;
-    __shared__ cpx<R> tw[N];
-    __shared__ cpx<R> buf[NG][LB];
-    const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
-    load_roots<R, N>(tw, a.tw);
-    __syncthreads();
-    const int np = a.NL * a.NZ2, K = a.nkx - 1;
-    const int pa = 2 * (blockIdx.x * NG + g), pb = pa + 1;
-    const cpx<R> *Z = reinterpret_cast<const cpx<R> *>(a.in);
-    cpx<R> x[MX];
-    sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
-    if (t < N1 && pa < np) {
-        const cpx<R> *A = Z + (size_t)pa * a.nkx;
-        const cpx<R> *Bv = pb < np ? Z + (size_t)pb * a.nkx : nullptr;
-        sfor<0, N2>([&](auto n2) {
-            const int k = t + N1 * decltype(n2)::value;
-            x[n2] = herm_pack(A, Bv, k, N, K);
-            // coarse grid, NXS = N/2: the Nyquist coefficient doubled (transforms.cpp:576-578)
-            if (a.coarse && 2 * k == N) x[n2] = {R(2) * x[n2].x, R(2) * x[n2].y};
-        });
-    }
-    two_pass<R, N1, N2, +1>(x, t, tw, buf[g], wsync);
-    if (t < N2) {
-        sfor<0, N1>([&](auto k1) {
-            const int n = t + N2 * decltype(k1)::value;
-            if (pa < np) {
-                const int l = pa / a.NZ2, iz = pa - l * a.NZ2;
-                a.phys[((size_t)iz * a.NL + l) * N + n] = double(x[k1].x);
-            }
-            if (pb < np) {
-                const int l = pb / a.NZ2, iz = pb - l * a.NZ2;
-                a.phys[((size_t)iz * a.NL + l) * N + n] = double(x[k1].y);
-            }
-        });
-    }
-}
-
-template <typename R, int N1, int N2>
-__global__ void __launch_bounds__(64) k_xfwd_phys_rf(XArgs a) {
-    using Gm = Geo<N1, N2>;
-    constexpr int N = Gm::N, MX = Gm::MX, G = Gm::G, NG = Gm::NG, LB = Gm::LB;
-    __shared__ cpx<R> tw[N];
-    __shared__ cpx<R> buf[NG][LB];
-    const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
-    load_roots<R, N>(tw, a.tw);
-    __syncthreads();
-    const int np = a.NL * a.NZ2, K = a.nkx - 1;
-    const int pa = 2 * (blockIdx.x * NG + g), pb = pa + 1;
-    cpx<R> x[MX];
-    sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
-    if (t < N2) {
-        sfor<0, N1>([&](auto j) {
-            const int n = t + N2 * decltype(j)::value;
-            R re = R(0), im = R(0);
-            if (pa < np) {
-                const int l = pa / a.NZ2, iz = pa - l * a.NZ2;
-                re = R(a.phys[((size_t)iz * a.NL + l) * N + n]);
-            }
-            if (pb < np) {
-                const int l = pb / a.NZ2, iz = pb - l * a.NZ2;
-                im = R(a.phys[((size_t)iz * a.NL + l) * N + n]);
-            }
-            x[j] = {re, im};
-        });
-    }
-    two_pass<R, N2, N1, -1>(x, t, tw, buf[g], wsync);
-    cpx<R> *B = buf[g];
-    if (t < N1) sfor<0, N2>([&](auto k1) { B[t + N1 * decltype(k1)::value] = x[k1]; });
-    wsync();
-    const R half = R(0.5) / R(N);
-    cpx<R> *ZN = reinterpret_cast<cpx<R> *>(a.out);
-    for (int k = t; k <= K; k += G) {
-        const cpx<R> f = B[k], gm = conjc(B[k == 0 ? 0 : N - k]);
-        const cpx<R> s = f + gm, d = f - gm;
-        // coarse grid, NXS = N/2: the Nyquist coefficient halved (transforms.cpp:496-497)
-        const R hk = (a.coarse && 2 * k == N) ? R(0.5) * half : half;
-        if (pa < np) ZN[zline_index(pa, k, a.nkx, a.NZ2)] = {hk * s.x, hk * s.y};
-        if (pb < np) ZN[zline_index(pb, k, a.nkx, a.NZ2)] = {hk * d.y, -hk * d.x};
-    }
-}
-
 // ------------------------------------------------------------------ z stages --
 // Backward: a block owns KB (16, or 8 for the largest lengths) consecutive kx lines of one
 // (field, l), one lane group per line; its output (Z[l][iz][kx], kx contiguous) goes through an LDS
@@ -558,16 +472,6 @@ template <typename R, int N1, int N2> static void go_xprod(const XArgs &a, hipSt
     using Gm = Geo<N1, N2>;
     hipLaunchKernelGGL((k_xprod_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + Gm::NG - 1) / Gm::NG), dim3(64), 0, st, a);
 }
-template <typename R, int N1, int N2> static void go_xbwd(const XArgs &a, hipStream_t st) {
-    using Gm = Geo<N1, N2>;
-    hipLaunchKernelGGL((k_xbwd_phys_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + 2 * Gm::NG - 1) / (2 * Gm::NG)), dim3(64), 0,
-                       st, a);
-}
-template <typename R, int N1, int N2> static void go_xfwd(const XArgs &a, hipStream_t st) {
-    using Gm = Geo<N1, N2>;
-    hipLaunchKernelGGL((k_xfwd_phys_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + 2 * Gm::NG - 1) / (2 * Gm::NG)), dim3(64), 0,
-                       st, a);
-}
 template <typename R, int N1, int N2> static void go_zbwd(const ZArgs &a, int nf, hipStream_t st) {
     if constexpr (N1 % 2 == 0 && N2 % 2 == 0) {
         if (a.pair) {
@@ -606,18 +510,6 @@ bool launch_xprod_rf(const XArgs &a, bool fp32, hipStream_t st) {
     const int n = a.plan.n;
 #define X(NN, A, B) case NN: if (fp32) go_xprod<float, A, B>(a, st); else go_xprod<double, A, B>(a, st); return true;
     switch (n) { CDNS_RF_SIZES(X) X(384, 16, 24) default: return false; }
-#undef X
-}
-bool launch_xbwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st) {
-    const int n = a.plan.n;
-#define X(NN, A, B) case NN: if (fp32) go_xbwd<float, A, B>(a, st); else go_xbwd<double, A, B>(a, st); return true;
-    switch (n) { CDNS_RF_SIZES(X) default: return false; }
-#undef X
-}
-bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st) {
-    const int n = a.plan.n;
-#define X(NN, A, B) case NN: if (fp32) go_xfwd<float, A, B>(a, st); else go_xfwd<double, A, B>(a, st); return true;
-    switch (n) { CDNS_RF_SIZES(X) default: return false; }
 #undef X
 }
 bool launch_zbwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st) {
