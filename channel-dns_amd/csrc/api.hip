@@ -207,6 +207,8 @@ struct cdns_ctx {
     void *ctwz = nullptr, *ctwx = nullptr;
     FftPlan cpz{}, cpx{};
     int *cflags = nullptr;
+    double *hsums = nullptr; // pinned host copies of csums and cflags
+    int *hflags = nullptr;
     std::vector<double> cc_weights; // Clenshaw-Curtis weights / 2 (diagnostics.cpp:17-33)
 
     // workspaces
@@ -459,8 +461,11 @@ void ensure_coarse(cdns_ctx *c) {
     c->ctwz = up_tw(g.NZ);
     c->ctwx = up_tw(g.NX);
     c->cphys = c->alloc<double>(5 * (size_t)g.NZ * NLc * g.NX);
-    c->csums = c->alloc<double>((size_t)NLc * kPlaneSums);
-    c->cflags = c->alloc<int>(std::max(NLc, 256));
+    const size_t ns = (size_t)NLc * moment_parts(NLc);
+    c->csums = c->alloc<double>(ns * kPlaneSums);
+    c->cflags = c->alloc<int>(4 * kFiniteBlocks + ns);
+    CDNS_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->hsums), ns * kPlaneSums * sizeof(double), hipHostMallocDefault));
+    CDNS_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->hflags), (4 * kFiniteBlocks + ns) * sizeof(int), hipHostMallocDefault));
     // Clenshaw-Curtis weights on [-1, 1] over height 2 (diagnostics.cpp:17-33)
     const int n = g.NY;
     const double pi = std::acos(-1.0);
@@ -488,6 +493,7 @@ YArgs yargs_coarse(cdns_ctx *c) {
     a.YS = (size_t)(c->g.NY + 1) * c->g.NQ;
     return a;
 }
+size_t coarse_points(const cdns_ctx *c) { return (size_t)c->g.NZ * (c->g.NY + 1) * c->g.NX; }
 size_t coarse_zs(const cdns_ctx *c) { return (size_t)(c->g.NY + 1) * c->g.NZ * c->g.nkx; }
 ZArgs zargs_coarse(cdns_ctx *c, const void *in, void *out) {
     const size_t ys = (size_t)(c->g.NY + 1) * c->g.NQ;
@@ -510,22 +516,32 @@ XArgs xargs_coarse(cdns_ctx *c, const void *in, void *out, double *phys) {
     a.phys = phys;
     return a;
 }
-// spectral plane -> coarse physical field [iz][iy][ix] (device)
-void coarse_backward(cdns_ctx *c, const zd *plane, double *phys) {
+// spectral planes -> coarse physical fields [iz][iy][ix] (device), field f at phys + f * coarse_points: as
+// many fields per launch as the product-grid workspaces hold (a launch for one field leaves most of the
+// device idle)
+void coarse_backward(cdns_ctx *c, const zd *const *planes, int n, double *phys) {
     ensure_coarse(c);
-    YArgs a = yargs_coarse(c);
-    a.spec[0] = plane;
-    {
-        Launch L(c, "coarse_y_backward");
-        launch_ybwd(a, 1, false, c->st);
-    }
-    {
-        Launch L(c, "coarse_z_backward");
-        launch_zbwd(zargs_coarse(c, c->Ybuf, c->Zbuf), 1, false, c->st);
-    }
-    {
-        Launch L(c, "coarse_x_backward");
-        launch_xbwd_phys(xargs_coarse(c, c->Zbuf, nullptr, phys), 1, false, c->st);
+    const Geometry &g = c->g;
+    YArgs y = yargs_coarse(c);
+    const size_t room_y = 6 * g.YS * c->esz / (y.YS * sizeof(zd)), room_z = 6 * g.ZS * c->esz / (coarse_zs(c) * sizeof(zd));
+    const int batch = (int)std::max<size_t>(1, std::min<size_t>({room_y, room_z, 6}));
+    for (int f0 = 0; f0 < n; f0 += batch) {
+        const int nf = std::min(batch, n - f0);
+        for (int f = 0; f < nf; ++f) y.spec[f] = planes[f0 + f];
+        {
+            Launch L(c, "coarse_y_backward");
+            launch_ybwd(y, nf, false, c->st);
+        }
+        {
+            Launch L(c, "coarse_z_backward");
+            launch_zbwd(zargs_coarse(c, c->Ybuf, c->Zbuf), nf, false, c->st);
+        }
+        XArgs x = xargs_coarse(c, c->Zbuf, nullptr, phys + (size_t)f0 * coarse_points(c));
+        x.phys_fs = coarse_points(c);
+        {
+            Launch L(c, "coarse_x_backward");
+            launch_xbwd_phys(x, nf, false, c->st);
+        }
     }
 }
 // coarse physical field (device) -> spectral plane
@@ -549,29 +565,25 @@ void coarse_forward(cdns_ctx *c, const double *phys, zd *plane) {
         launch_yfwd(a, 1, false, c->st);
     }
 }
-size_t coarse_points(const cdns_ctx *c) { return (size_t)c->g.NZ * (c->g.NY + 1) * c->g.NX; }
-// FieldIO::to_physical (field_io.cpp:199-220) of the state into cphys[0..3] (u, v, w, pressure);
-// returns whether every retained spectral coefficient is finite
-bool state_to_physical(cdns_ctx *c) {
+// FieldIO::to_physical (field_io.cpp:199-220) of the state into cphys[0..3] (u, v, w, pressure) and, with a
+// plane div, its field into cphys[4].  With check: the finite flags of the four state planes' blocks go to
+// the pinned host buffer, valid after the next stream synchronisation (state_finite).
+void state_to_physical(cdns_ctx *c, bool check, const zd *div = nullptr) {
     ensure_coarse(c);
-    const zd *src[4] = {c->u[0], c->u[1], c->u[2], c->P_};
-    for (int k = 0; k < 4; ++k) coarse_backward(c, src[k], c->cphys + k * coarse_points(c));
-    int ok = 1;
-    const int nb = 256;
-    std::vector<int> flags(nb);
-    for (int k = 0; k < 4; ++k) {
-        launch_planes_finite(src[k], 1, c->g.NQ, c->g.JS, c->g.NYS, c->cflags, nb, c->st);
-        CDNS_HIP(hipMemcpyAsync(flags.data(), c->cflags, nb * sizeof(int), hipMemcpyDeviceToHost, c->st));
-        CDNS_HIP(hipStreamSynchronize(c->st));
-        for (int f : flags) ok &= f;
-    }
-    return ok != 0;
+    const zd *src[5] = {c->u[0], c->u[1], c->u[2], c->P_, div};
+    coarse_backward(c, src, div ? 5 : 4, c->cphys);
+    if (!check) return;
+    launch_planes_finite(src, 4, c->g.NQ, c->g.JS, c->g.NYS, c->cflags, kFiniteBlocks, c->st);
+    CDNS_HIP(hipMemcpyAsync(c->hflags, c->cflags, 4 * kFiniteBlocks * sizeof(int), hipMemcpyDeviceToHost, c->st));
 }
-// Statistics::reduce over cphys (and the plane sum of div^2 when with_div) into host sums
+bool state_finite(const cdns_ctx *c) {
+    return std::all_of(c->hflags, c->hflags + 4 * kFiniteBlocks, [](int f) { return f != 0; });
+}
+// Statistics::reduce over cphys (and the plane sum of div^2 when with_div) into host sums; synchronises
 void plane_moments(cdns_ctx *c, bool higher, bool with_div, std::vector<double> &sums, std::vector<int> &finite) {
     const Geometry &g = c->g;
-    const int NLc = g.NY + 1;
-    const size_t np = coarse_points(c);
+    const int NLc = g.NY + 1, parts = moment_parts(NLc);
+    const size_t np = coarse_points(c), ns = (size_t)NLc * parts;
     DiagArgs a{};
     a.pu = c->cphys;
     a.pv = c->cphys + np;
@@ -581,18 +593,26 @@ void plane_moments(cdns_ctx *c, bool higher, bool with_div, std::vector<double> 
     a.NX = g.NX;
     a.NZ = g.NZ;
     a.NL = NLc;
+    a.parts = parts;
     a.higher = higher ? 1 : 0;
     a.sums = c->csums;
-    a.finite = c->cflags;
+    a.finite = c->cflags + 4 * kFiniteBlocks;
     {
         Launch L(c, "plane_moments");
         launch_plane_moments(a, c->st);
     }
-    sums.resize((size_t)NLc * kPlaneSums);
-    finite.resize(NLc);
-    CDNS_HIP(hipMemcpyAsync(sums.data(), c->csums, sums.size() * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    CDNS_HIP(hipMemcpyAsync(finite.data(), c->cflags, NLc * sizeof(int), hipMemcpyDeviceToHost, c->st));
+    int *const hf = c->hflags + 4 * kFiniteBlocks;
+    CDNS_HIP(hipMemcpyAsync(c->hsums, c->csums, ns * kPlaneSums * sizeof(double), hipMemcpyDeviceToHost, c->st));
+    CDNS_HIP(hipMemcpyAsync(hf, a.finite, ns * sizeof(int), hipMemcpyDeviceToHost, c->st));
     CDNS_HIP(hipStreamSynchronize(c->st));
+    sums.assign((size_t)NLc * kPlaneSums, 0.0);
+    finite.assign(NLc, 1);
+    for (int iy = 0; iy < NLc; ++iy)
+        for (int p = 0; p < parts; ++p) { // the parts of a plane in a fixed order
+            const size_t e = (size_t)iy * parts + p;
+            for (int m = 0; m < kPlaneSums; ++m) sums[(size_t)iy * kPlaneSums + m] += c->hsums[e * kPlaneSums + m];
+            finite[iy] &= hf[e];
+        }
 }
 
 void curl_planes(cdns_ctx *c, zd *const *u, zd *const *w, zd *bcw) {
@@ -1407,6 +1427,8 @@ void cdns_destroy(cdns_ctx *c) {
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->hz_ck) (void)hipFree(c->hz_ck);
     if (c->hz_seg) (void)hipFree(c->hz_seg);
+    if (c->hsums) (void)hipHostFree(c->hsums);
+    if (c->hflags) (void)hipHostFree(c->hflags);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
 }
@@ -1505,7 +1527,8 @@ int cdns_xyzfft(cdns_ctx *c, char dir, double *phys, double *spec, int stride, i
         if (dir == 'B') {
             zd *pl[1] = {c->scr[0]};
             ref_to_planes(c, spec, stride, 1, g.nj, pl, where, g.JS);
-            coarse_backward(c, c->scr[0], dphys);
+            const zd *cp[1] = {c->scr[0]};
+            coarse_backward(c, cp, 1, dphys);
             if (where == CDNS_HOST)
                 CDNS_HIP(hipMemcpyAsync(phys, dphys, np * sizeof(double), hipMemcpyDeviceToHost, c->st));
         } else {
@@ -1524,13 +1547,13 @@ int cdns_xyzfft(cdns_ctx *c, char dir, double *phys, double *spec, int stride, i
 
 int cdns_to_physical(cdns_ctx *c, double *velocity, double *pressure, int *finite, int where) {
     try {
-        const bool ok = state_to_physical(c);
+        state_to_physical(c, finite != nullptr);
         const size_t np = coarse_points(c);
         const hipMemcpyKind kind = where == CDNS_HOST ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
         if (velocity) CDNS_HIP(hipMemcpyAsync(velocity, c->cphys, 3 * np * sizeof(double), kind, c->st));
         if (pressure) CDNS_HIP(hipMemcpyAsync(pressure, c->cphys + 3 * np, np * sizeof(double), kind, c->st));
         CDNS_HIP(hipStreamSynchronize(c->st));
-        if (finite) *finite = ok ? 1 : 0;
+        if (finite) *finite = state_finite(c) ? 1 : 0;
         return 0;
     } catch (const std::exception &e) {
         return fail(c, e);
@@ -1539,7 +1562,7 @@ int cdns_to_physical(cdns_ctx *c, double *velocity, double *pressure, int *finit
 
 int cdns_plane_moments(cdns_ctx *c, int higher, double *sums, int *finite) {
     try {
-        state_to_physical(c);
+        state_to_physical(c, false);
         std::vector<double> s;
         std::vector<int> f;
         plane_moments(c, higher != 0, false, s, f);
@@ -1557,7 +1580,7 @@ int cdns_plane_moments(cdns_ctx *c, int higher, double *sums, int *finite) {
 int cdns_diagnostics(cdns_ctx *c, double out[3], int *finite) {
     try {
         const Geometry &g = c->g;
-        bool ok = state_to_physical(c);
+        ensure_coarse(c);
         DiagArgs d{};
         d.u = c->u[0];
         d.v = c->u[1];
@@ -1573,10 +1596,11 @@ int cdns_diagnostics(cdns_ctx *c, double out[3], int *finite) {
             Launch L(c, "divergence");
             launch_divergence(d, g.E, c->st);
         }
-        coarse_backward(c, c->scr[0], c->cphys + 4 * coarse_points(c));
+        state_to_physical(c, true, c->scr[0]);
         std::vector<double> s;
         std::vector<int> f;
         plane_moments(c, false, true, s, f);
+        bool ok = state_finite(c);
         // Diagnostics::evaluate (diagnostics.cpp:39-75)
         const double inv_plane = 1.0 / ((double)g.NX * g.NZ);
         double ekt = 0.0, tke = 0.0, div2 = 0.0;

@@ -212,11 +212,15 @@ struct DiagArgs {
     int NQ, nzk, JS, ny;
     const double *pu, *pv, *pw, *pp, *pdiv; // physical [iz][iy][ix]; pdiv may be null
     int NX, NZ, NL, higher;
-    double *sums; // [NL][kPlaneSums]
-    int *finite;  // [NL]
+    int parts;    // blocks per plane (moment_parts)
+    double *sums; // [NL][parts][kPlaneSums]
+    int *finite;  // [NL][parts]
 };
+int moment_parts(int NL);
+constexpr int kFiniteBlocks = 256; // blocks (and flags) per plane of the finiteness check
 void launch_divergence(const DiagArgs &a, int E, hipStream_t st);
-void launch_planes_finite(const zd *planes, size_t nplanes, int NQ, int JS, int ny, int *flags, int nblocks,
+// n <= 4 planes; flags[plane * nblocks + b]
+void launch_planes_finite(const zd *const *planes, int n, int NQ, int JS, int ny, int *flags, int nblocks,
                           hipStream_t st);
 void launch_plane_moments(const DiagArgs &a, hipStream_t st);
 
