@@ -208,8 +208,8 @@ class Channel:
     # FieldIO::to_physical: (velocity [3][NZ][NY+1][NX], pressure [NZ][NY+1][NX], finite)
     def to_physical(self):
         m = self.cfg
-        vel = np.zeros((3, m["NZ"], m["NY"] + 1, m["NX"]), np.float64)
-        pr = self.coarse_phys()
+        vel = np.empty((3, m["NZ"], m["NY"] + 1, m["NX"]), np.float64)  # every value is written
+        pr = np.empty(vel.shape[1:], np.float64)
         fin = ctypes.c_int(0)
         self._check(lib().cdns_to_physical(self._h, _ptr(vel), _ptr(pr), ctypes.byref(fin), HOST))
         return vel, pr, bool(fin.value)
@@ -282,14 +282,17 @@ class Channel:
     def set_state(self, name, data):
         if isinstance(data, np.ndarray):
             arr = self._shape(name)
-            arr[...] = data
+            if data.shape == arr.shape and data.dtype == arr.dtype and data.flags.c_contiguous:
+                arr = data
+            else:
+                arr[...] = data
             self._check(lib().cdns_set_state(self._h, STATE[name], _ptr(arr), HOST))
         else:
             self._check(lib().cdns_set_state(self._h, STATE[name], _ptr(data), DEVICE))
 
     def get_state(self, name, out=None):
         if out is None:
-            arr = self._shape(name)
+            arr = np.empty_like(self._shape(name))  # every value is written
             self._check(lib().cdns_get_state(self._h, STATE[name], _ptr(arr), HOST))
             return arr
         self._check(lib().cdns_get_state(self._h, STATE[name], _ptr(out), DEVICE))

@@ -1032,13 +1032,16 @@ void ref_to_planes(cdns_ctx *c, const double *src, int stride, int ncomp, int nr
     const zd *dev = reinterpret_cast<const zd *>(src);
     int dstride = stride;
     if (where == CDNS_HOST) {
-        // gather the (possibly strided) components into the staging buffer
-        std::vector<zd> tmp(n * ncomp);
-        const zd *h = reinterpret_cast<const zd *>(src);
-        for (size_t e = 0; e < n; ++e)
-            for (int k = 0; k < ncomp; ++k) tmp[e * ncomp + k] = h[e * stride + k];
         zd *stage = nrow == 2 ? c->bnd_stage : c->ref_stage;
-        CDNS_HIP(hipMemcpyAsync(stage, tmp.data(), tmp.size() * sizeof(zd), hipMemcpyHostToDevice, c->st));
+        const zd *h = reinterpret_cast<const zd *>(src);
+        std::unique_ptr<zd[]> tmp;
+        if (stride != ncomp) { // gather the strided components
+            tmp.reset(new zd[n * ncomp]);
+            for (size_t e = 0; e < n; ++e)
+                for (int k = 0; k < ncomp; ++k) tmp[e * ncomp + k] = h[e * stride + k];
+            h = tmp.get();
+        }
+        CDNS_HIP(hipMemcpyAsync(stage, h, n * ncomp * sizeof(zd), hipMemcpyHostToDevice, c->st));
         CDNS_HIP(hipStreamSynchronize(c->st));
         dev = stage;
         dstride = ncomp;
@@ -1081,12 +1084,14 @@ void planes_to_ref(cdns_ctx *c, const zd *const *planes, int ncomp, int nrow, do
         Launch L(c, "layout_out");
         launch_planes_to_ref(a, c->st);
     }
-    std::vector<zd> tmp(n * ncomp);
-    CDNS_HIP(hipMemcpyAsync(tmp.data(), stage, tmp.size() * sizeof(zd), hipMemcpyDeviceToHost, c->st));
-    CDNS_HIP(hipStreamSynchronize(c->st));
     zd *h = reinterpret_cast<zd *>(dst);
-    for (size_t e = 0; e < n; ++e)
-        for (int k = 0; k < ncomp; ++k) h[e * stride + k] = tmp[e * ncomp + k];
+    std::unique_ptr<zd[]> tmp;
+    if (stride != ncomp) tmp.reset(new zd[n * ncomp]);
+    CDNS_HIP(hipMemcpyAsync(tmp ? tmp.get() : h, stage, n * ncomp * sizeof(zd), hipMemcpyDeviceToHost, c->st));
+    CDNS_HIP(hipStreamSynchronize(c->st));
+    if (tmp)
+        for (size_t e = 0; e < n; ++e)
+            for (int k = 0; k < ncomp; ++k) h[e * stride + k] = tmp[e * ncomp + k];
 }
 
 int fail(cdns_ctx *c, const std::exception &e) {
