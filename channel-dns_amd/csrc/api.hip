@@ -753,19 +753,35 @@ void setup(cdns_ctx *c, double g_v) {
     const Geometry &g = c->g;
     c->g_v = g_v;
     {
+        AdArgs a{};
+        a.WAVX = c->WAVX;
+        a.WAVZ = c->WAVZ;
+        a.WL = c->WL;
+        a.WD = c->WD;
+        a.WR = c->WR;
+        a.g[0] = c->cfg.G_pre;
+        a.g[1] = g_v;
+        a.ny = g.NYS;
+        a.JS = g.JS;
+        a.NQ = g.NQ;
+        a.nzk = g.nzk;
+        a.ad[0] = c->ad_p;
+        a.ad[1] = c->ad_v;
+        a.wn[0] = c->wn_p;
+        a.wn[1] = c->wn_v;
         Launch L(c, "setup_ad");
-        launch_build_ad(c->WAVX, c->WAVZ, c->WL, c->WD, c->WR, c->cfg.G_pre, g.NYS, g.JS, g.NQ, g.nzk, c->ad_p,
-                        c->wn_p, c->st);
-        launch_build_ad(c->WAVX, c->WAVZ, c->WL, c->WD, c->WR, g_v, g.NYS, g.JS, g.NQ, g.nzk, c->ad_v, c->wn_v, c->st);
+        launch_build_ad(a, c->st);
     }
     c->pa = 1.0;
     c->pb = 0.0;
-    for (int i = 0; i < 2; ++i) {
+    {
         SolveArgs a = solve_args(c, MODE_INFLUENCE);
-        a.influence_index = i;
-        a.P = c->PI[i];
-        for (int k = 0; k < 3; ++k) a.V[k] = c->VI[i][k];
-        a.div_out = c->ID[i];
+        for (int i = 0; i < 2; ++i) {
+            a.infl_P[i] = c->PI[i];
+            for (int k = 0; k < 3; ++k) a.infl_V[i][k] = c->VI[i][k];
+            a.infl_div[i] = c->ID[i];
+            for (int k = 0; k < 3; ++k) a.ctab_infl[i][k] = c->ctab[2 * k + i]; // PIr, VIv, VIf
+        }
         Launch L(c, "setup_influence");
         launch_solve(a, g.E, c->st);
     }
@@ -779,14 +795,9 @@ void setup(cdns_ctx *c, double g_v) {
         a.P = c->PB;
         for (int k = 0; k < 3; ++k) a.V[k] = c->VB[k];
         a.sig_out = c->SIG0;
+        for (int k = 0; k < 3; ++k) a.ctab_b[k] = c->ctab[6 + k]; // PBr, VBv, VBf
         Launch L(c, "setup_bproblem");
         launch_solve(a, g.E, c->st);
-    }
-    if (c->compact) {
-        SolveArgs a = solve_args(c, MODE_STEP);
-        Launch L(c, "setup_compact");
-        launch_compact_tables(a, c->ctab[0], c->ctab[1], c->ctab[2], c->ctab[3], c->ctab[4], c->ctab[5], c->ctab[6],
-                              c->ctab[7], c->ctab[8], c->st);
     }
     c->pa = c->cfg.a_pre0;
     c->pb = c->cfg.b_pre0;

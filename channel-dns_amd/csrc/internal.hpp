@@ -157,7 +157,6 @@ struct SolveArgs {
     const zd *bcw;   // step: curl part of the pressure wall condition [q][2]
     zd *bc_prev;     // step: in B^{n-1}, out B^n [q][2]
     zd *bc_ext;      // step: out b0 B^n + b1 B^{n-1} [q][2]
-    int influence_index;
     int correct, sigma;
     // tables
     const double *ad_p, *ad_v;
@@ -172,7 +171,9 @@ struct SolveArgs {
     int grad_pre;
     // outputs
     zd *P, *V[3];
-    zd *div_out;  // influence: raw wall divergence [q][2]
+    // influence, per wall: pressure, velocity, raw wall divergence [q][2], compact tables (P, v, phi)
+    zd *infl_P[2], *infl_V[2][3], *infl_div[2];
+    double *ctab_infl[2][3], *ctab_b[3]; // compact: written with the responses (influence, B problem)
     zd *sig_out;  // b problem: sigma0 [q][2]
     double *flow; // step: dpdx, dpdz
 };
@@ -225,12 +226,14 @@ void launch_planes_finite(const zd *const *planes, int n, int NQ, int JS, int ny
 void launch_plane_moments(const DiagArgs &a, hipStream_t st);
 
 void launch_solve(const SolveArgs &a, int E, hipStream_t st);
-// real tables of the compact form from the complex setup tables
-void launch_compact_tables(const SolveArgs &a, double *PIr0, double *PIr1, double *VIv0, double *VIv1,
-                           double *VIf0, double *VIf1, double *PBr, double *VBv, double *VBf, hipStream_t st);
-void launch_build_ad(const double *WAVX, const double *WAVZ, const double *WL, const double *WD,
-                     const double *WR, double g, int ny, int JS, int NQ, int nzk, double *ad,
-                     double *wn, hipStream_t st);
+// ad and wn tables of the pressure (0) and the velocity (1) operator
+struct AdArgs {
+    const double *WAVX, *WAVZ, *WL, *WD, *WR;
+    double g[2];
+    int ny, JS, NQ, nzk;
+    double *ad[2], *wn[2];
+};
+void launch_build_ad(const AdArgs &a, hipStream_t st);
 void launch_normalize_influence(zd *ID0, zd *ID1, int NQ, int root_q, double aV1, hipStream_t st);
 void launch_pg_response(const double *WAVX, const double *WAVZ, const double *WL, const double *WD,
                         const double *WR, const double *ad_v, double g_v, double Re, const double *aV,

@@ -120,6 +120,24 @@ __device__ void tau_solve(const zd (&r)[NR][NE], zd (&out)[NR][NE], const double
     sp::prefix_affine_c<NE, NR>(aa, bb, out, lane);
 }
 
+// Compact form of one response column (P, v real; u = i kx phi, w = i kz phi): the influence and B
+// responses come from real wall data and real operators, so P and v are real and u, w share one real
+// phi when u and w share their wall conditions (eqsolve_pv.cpp:266-303, 452-477).  Written by the solve
+// that holds the column: as a pass of its own it read the nine complex tables again (Re_tau=180, 42 us
+// per setup).
+template <int NE>
+__device__ inline void store_compact(double *const (&t)[3], size_t off, int lane, int ny, double kx, double kz,
+                                     const zd (&P)[NE], const zd (&V)[3][NE]) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+        const int j = sp::jof<NE>(lane, e);
+        if (j > ny) continue;
+        t[0][off + j] = P[e].x;
+        t[1][off + j] = V[1][e].x;
+        t[2][off + j] = kx != 0.0 ? V[0][e].y / kx : (kz != 0.0 ? V[2][e].y / kz : 0.0);
+    }
+}
+
 // Fused coupled solve of one (kx,kz) pair: EqSolvePV::solve_modes (eqsolve_pv.cpp:311-450),
 // with the step's RHS assembly (simulation.cpp:144-160), the nonlinear pressure wall condition
 // (timestepper.cpp:26-43), correct_zero_mode (timestepper.cpp:60-68) and correct_flow
@@ -239,8 +257,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE == 
         plo[0] = a.pbc[(size_t)q * 2 + 0];
         pup[0] = a.pbc[(size_t)q * 2 + 1];
     } else if constexpr (mode == MODE_INFLUENCE) {
-        plo[0] = {(double)(1 - a.influence_index), 0.0};
-        pup[0] = {(double)a.influence_index, 0.0};
+        plo[0] = {(double)(1 - (int)blockIdx.y), 0.0};
+        pup[0] = {(double)blockIdx.y, 0.0};
     }
     zd vlo[3], vup[3];
 #pragma unroll
@@ -312,13 +330,15 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE == 
         div1 = {t[2], t[3]};
     }
     if constexpr (mode == MODE_INFLUENCE) {
+        const int i = blockIdx.y;
         if (lane == 0) {
-            a.div_out[(size_t)q * 2 + 0] = div0;
-            a.div_out[(size_t)q * 2 + 1] = div1;
+            a.infl_div[i][(size_t)q * 2 + 0] = div0;
+            a.infl_div[i][(size_t)q * 2 + 1] = div1;
         }
-        sp::store_col<NE>(a.P + off, lane, ny, pc[0]);
+        sp::store_col<NE>(a.infl_P[i] + off, lane, ny, pc[0]);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) sp::store_col<NE>(a.V[k] + off, lane, ny, vc[k]);
+        for (int k = 0; k < 3; ++k) sp::store_col<NE>(a.infl_V[i][k] + off, lane, ny, vc[k]);
+        if (a.compact) store_compact<NE>(a.ctab_infl[i], off, lane, ny, kx, kz, pc[0], vc);
         return;
     }
 
@@ -457,6 +477,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE == 
             a.sig_out[(size_t)q * 2 + 1] = s1;
         }
     }
+    if constexpr (mode == MODE_BPROBLEM)
+        if (a.compact) store_compact<NE>(a.ctab_b, off, lane, ny, kx, kz, P, V);
     sp::store_col<NE>(a.P + off, lane, ny, P);
 #pragma unroll
     for (int k = 0; k < 3; ++k) sp::store_col<NE>(a.V[k] + off, lane, ny, V[k]);
@@ -470,7 +492,9 @@ template <int NE> static void launch_solve_mode(const SolveArgs &a, hipStream_t 
         else hipLaunchKernelGGL((k_solve<NE, MODE_STEP>), grid, block, 0, st, a);
         break;
     case MODE_GIVEN: hipLaunchKernelGGL((k_solve<NE, MODE_GIVEN>), grid, block, 0, st, a); break;
-    case MODE_INFLUENCE: hipLaunchKernelGGL((k_solve<NE, MODE_INFLUENCE>), grid, block, 0, st, a); break;
+    case MODE_INFLUENCE: // both walls
+        hipLaunchKernelGGL((k_solve<NE, MODE_INFLUENCE>), dim3(grid.x, 2), block, 0, st, a);
+        break;
     case MODE_BPROBLEM: hipLaunchKernelGGL((k_solve<NE, MODE_BPROBLEM>), grid, block, 0, st, a); break;
     default: throw std::runtime_error("unknown solve mode");
     }
@@ -483,61 +507,46 @@ void launch_solve(const SolveArgs &a, int E, hipStream_t st) {
     else throw std::runtime_error("unsupported column length");
 }
 
-// Compact tables: the influence and B responses come from real wall data and real operators,
-// so P and v are real and u, w are i kx phi, i kz phi with one real phi when u and w share their
-// wall conditions (eqsolve_pv.cpp:266-303, 452-477).
-__global__ void k_compact_tables(SolveArgs a, double *PIr0, double *PIr1, double *VIv0, double *VIv1, double *VIf0,
-                                 double *VIf1, double *PBr, double *VBv, double *VBf) {
-    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (size_t)a.NQ * a.JS) return;
-    const int q = (int)(e / a.JS);
-    const int kxi = q / a.nzk, kzi = q - kxi * a.nzk;
-    const double kx = a.WAVX[kxi], kz = a.WAVZ[kzi];
-    auto phi = [&](const zd *u, const zd *w) {
-        if (kx != 0.0) return u[e].y / kx;
-        if (kz != 0.0) return w[e].y / kz;
-        return 0.0;
-    };
-    PIr0[e] = a.PI[0][e].x;
-    PIr1[e] = a.PI[1][e].x;
-    VIv0[e] = a.VI[0][1][e].x;
-    VIv1[e] = a.VI[1][1][e].x;
-    VIf0[e] = phi(a.VI[0][0], a.VI[0][2]);
-    VIf1[e] = phi(a.VI[1][0], a.VI[1][2]);
-    PBr[e] = a.PB[e].x;
-    VBv[e] = a.VB[1][e].x;
-    VBf[e] = phi(a.VB[0], a.VB[2]);
-}
-void launch_compact_tables(const SolveArgs &a, double *PIr0, double *PIr1, double *VIv0, double *VIv1,
-                           double *VIf0, double *VIf1, double *PBr, double *VBv, double *VBf, hipStream_t st) {
-    const size_t n = (size_t)a.NQ * a.JS;
-    hipLaunchKernelGGL(k_compact_tables, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, a, PIr0, PIr1, VIv0,
-                       VIv1, VIf0, VIf1, PBr, VBv, VBf);
-}
-
-// build_wn_ad (eqsolve_pv.cpp:148-168): continued-fraction recurrence, one thread per pair.
-__global__ void k_build_ad(const double *WAVX, const double *WAVZ, const double *WL, const double *WD,
-                           const double *WR, double g, int ny, int JS, int NQ, int nzk, double *ad, double *wn) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= NQ) return;
-    const int kxi = q / nzk, kzi = q - kxi * nzk;
-    const double w = -(WAVX[kxi] * WAVX[kxi] + WAVZ[kzi] * WAVZ[kzi] + g);
-    wn[q] = w;
-    double *col = ad + (size_t)q * JS;
-    col[0] = 0.0;
-    col[1] = 0.0;
-    col[ny] = 1.0 / (1.0 + WD[ny] * w);
-    col[ny - 1] = 1.0 / (1.0 + WD[ny - 1] * w);
-    for (int iy = ny - 2; iy >= 2; --iy) {
-        const double fc = WR[iy] * WL[iy + 2];
-        const double den = 1.0 + (WD[iy] - fc * w * col[iy + 2]) * w;
-        col[iy] = 1.0 / den;
+// build_wn_ad (eqsolve_pv.cpp:148-168) for the pressure and the velocity operator: a continued-fraction
+// recurrence down each parity chain of a column.  One wavefront carries 16 columns x 2 tables x 2 chains;
+// the chain's last value stays in a register and every 32 entries leave through LDS as whole runs.  Bound
+// by the dependent divisions (63 per chain at Re_tau=180).  With one thread per column, each step read the
+// entry two rows up back from memory: 82 us for both tables, AD_US so.
+constexpr int kAdCols = 16;
+__global__ void __launch_bounds__(64) k_build_ad(AdArgs a) {
+    __shared__ double tile[2 * kAdCols][33];
+    __shared__ double2 coef[256]; // WD(j), WR(j) WL(j+2)
+    const int lane = threadIdx.x, row = lane >> 1, p = lane & 1, tab = row / kAdCols;
+    const int q = blockIdx.x * kAdCols + row % kAdCols, ny = a.ny;
+    const bool on = q < a.NQ;
+    const int qc = on ? q : 0, kxi = qc / a.nzk, kzi = qc - kxi * a.nzk;
+    const double w = -(a.WAVX[kxi] * a.WAVX[kxi] + a.WAVZ[kzi] * a.WAVZ[kzi] + a.g[tab]);
+    if (on && p == 0) a.wn[tab][q] = w;
+    for (int j = lane; j <= ny; j += 64) coef[j] = double2{a.WD[j], j <= ny - 2 ? a.WR[j] * a.WL[j + 2] : 0.0};
+    __syncthreads();
+    double prev = 0.0; // entry iy + 2
+    for (int j0 = ny & ~31; j0 >= 0; j0 -= 32) {
+        double2 cf[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) cf[i] = coef[min(j0 + 2 * i + p, ny)];
+#pragma unroll
+        for (int i = 15; i >= 0; --i) {
+            const int iy = j0 + 2 * i + p;
+            // the chain starts at ny or ny - 1 with prev = 0: 1 / (1 + WD w)
+            const double fc = cf[i].y, den = 1.0 + (cf[i].x - fc * w * prev) * w;
+            prev = iy <= ny ? 1.0 / den : 0.0;
+            tile[row][2 * i + p] = iy >= 2 ? prev : 0.0;
+        }
+        __syncthreads();
+        for (int e = lane; e < 2 * kAdCols * 32; e += 64) {
+            const int r = e >> 5, j = j0 + (e & 31), qr = blockIdx.x * kAdCols + r % kAdCols;
+            if (qr < a.NQ && j <= ny) a.ad[r / kAdCols][(size_t)qr * a.JS + j] = tile[r][e & 31];
+        }
+        __syncthreads();
     }
 }
-void launch_build_ad(const double *WAVX, const double *WAVZ, const double *WL, const double *WD, const double *WR,
-                     double g, int ny, int JS, int NQ, int nzk, double *ad, double *wn, hipStream_t st) {
-    hipLaunchKernelGGL(k_build_ad, dim3((NQ + 127) / 128), dim3(128), 0, st, WAVX, WAVZ, WL, WD, WR, g, ny, JS, NQ,
-                       nzk, ad, wn);
+void launch_build_ad(const AdArgs &a, hipStream_t st) {
+    hipLaunchKernelGGL(k_build_ad, dim3((a.NQ + kAdCols - 1) / kAdCols), dim3(64), 0, st, a);
 }
 
 // build_influence_coefficients normalisation (eqsolve_pv.cpp:282-302).
