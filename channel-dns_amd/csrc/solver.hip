@@ -511,7 +511,7 @@ void launch_solve(const SolveArgs &a, int E, hipStream_t st) {
 // recurrence down each parity chain of a column.  One wavefront carries 16 columns x 2 tables x 2 chains;
 // the chain's last value stays in a register and every 32 entries leave through LDS as whole runs.  Bound
 // by the dependent divisions (63 per chain at Re_tau=180).  With one thread per column, each step read the
-// entry two rows up back from memory: 82 us for both tables, AD_US so.
+// entry two rows up back from memory: 82 us for both tables at Re_tau=180, 22 us so (between HIP events).
 constexpr int kAdCols = 16;
 __global__ void __launch_bounds__(64) k_build_ad(AdArgs a) {
     __shared__ double tile[2 * kAdCols][33];
