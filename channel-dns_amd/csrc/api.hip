@@ -420,18 +420,6 @@ void forward_zy(cdns_ctx *c, zd *const *planes, int n, const void *zin = nullptr
     }
 }
 
-// N = a x b (+ add) for spectral vector planes (a: 3 planes, b: 3 planes)
-void cross_planes(cdns_ctx *c, zd *const *a, zd *const *b, zd *const *out, zd *const *add = nullptr,
-                  bool out32 = false) {
-    const zd *f6[6] = {a[0], a[1], a[2], b[0], b[1], b[2]};
-    backward_yz(c, f6, 6);
-    {
-        Launch L(c, "x_product");
-        launch_xprod(xargs(c, c->Zbuf, c->ZNbuf, c->g.ZS, c->g.ZS, c->P), c->fp32, c->st);
-    }
-    forward_zy(c, out, 3, nullptr, add, out32);
-}
-
 // ------------------------------------------------------------- coarse grid ----
 // Transforms::channel_xyzfft (transforms.cpp:452-582): the base grid NX x (NY+1) x NZ of
 // to_physical, statistics and diagnostics, always in FP64, in the product-grid workspaces.
@@ -633,31 +621,22 @@ void curl_planes(cdns_ctx *c, zd *const *u, zd *const *w, zd *bcw) {
     launch_curl(a, c->g.E, c->st);
 }
 
-// TimeStepper::enqueue_nonlinear_term on the context's velocity planes
-void nonlinear_planes(cdns_ctx *c, zd *const *u, zd *const *nl, bool out32 = false) {
-    zd *const *add = c->body_on ? c->body : nullptr;
+// Velocity planes -> their six z-physical fields (u, curl u) in the context's Z buffer, and the curl part
+// of the pressure wall condition in bcw
+void synthesise(cdns_ctx *c, zd *const *u) {
+    bool done = false;
     if (c->ydct && c->ycurl) {
-        // DCT-I y backward of u with the curl formed per column: the six Y fields and the wall
-        // condition
+        // DCT-I y backward of u with the curl formed per column
         DctArgs a = dct_args(c);
         for (int k = 0; k < 3; ++k) a.spec[k] = u[k];
         a.nf = 6;
         a.curl = 1;
         a.bcw = c->bcw;
-        {
-            Launch L(c, "y_backward_curl");
-            if (!launch_ybwd_dct(a, c->fp32, c->st)) throw std::logic_error("no DCT y stage for this NY2");
-        }
-        backward_z(c, 6);
-        {
-            Launch L(c, "x_product");
-            launch_xprod(xargs(c, c->Zbuf, c->ZNbuf, c->g.ZS, c->g.ZS, c->P), c->fp32, c->st);
-        }
-        forward_zy(c, nl, 3, nullptr, add, out32);
-        return;
-    }
-    if (c->ymfma && c->ycurl) {
-        // y backward of u with the curl fused in: the six Y fields and the wall condition
+        Launch L(c, "y_backward_curl");
+        if (!launch_ybwd_dct(a, c->fp32, c->st)) throw std::logic_error("no DCT y stage for this NY2");
+        done = true;
+    } else if (c->ymfma && c->ycurl) {
+        // y backward of u with the curl fused in
         YArgs a = yargs(c);
         for (int k = 0; k < 3; ++k) a.spec[k] = u[k];
         a.coefd = c->ycoef_d;
@@ -666,23 +645,30 @@ void nonlinear_planes(cdns_ctx *c, zd *const *u, zd *const *nl, bool out32 = fal
         a.Re = c->cfg.Re;
         a.nzk = c->g.nzk;
         a.bcw = c->bcw;
-        bool done;
-        {
-            Launch L(c, "y_backward_curl");
-            done = launch_ybwd_curl(a, c->fp32, c->st);
-        }
-        if (done) {
-            backward_z(c, 6);
-            {
-                Launch L(c, "x_product");
-                launch_xprod(xargs(c, c->Zbuf, c->ZNbuf, c->g.ZS, c->g.ZS, c->P), c->fp32, c->st);
-            }
-            forward_zy(c, nl, 3, nullptr, add, out32);
-            return;
-        }
+        Launch L(c, "y_backward_curl");
+        done = launch_ybwd_curl(a, c->fp32, c->st);
+    }
+    if (done) {
+        backward_z(c, 6);
+        return;
     }
     curl_planes(c, u, c->om, c->bcw);
-    cross_planes(c, u, c->om, nl, add, out32);
+    const zd *f6[6] = {u[0], u[1], u[2], c->om[0], c->om[1], c->om[2]};
+    backward_yz(c, f6, 6);
+}
+// The product of the six z-physical fields in the Z buffer, analysed into planes (+ add)
+void product_forward(cdns_ctx *c, zd *const *out, zd *const *add, bool out32) {
+    {
+        Launch L(c, "x_product");
+        launch_xprod(xargs(c, c->Zbuf, c->ZNbuf, c->g.ZS, c->g.ZS, c->P), c->fp32, c->st);
+    }
+    forward_zy(c, out, 3, nullptr, add, out32);
+}
+
+// TimeStepper::enqueue_nonlinear_term on the context's velocity planes
+void nonlinear_planes(cdns_ctx *c, zd *const *u, zd *const *nl, bool out32 = false) {
+    synthesise(c, u);
+    product_forward(c, nl, c->body_on ? c->body : nullptr, out32);
 }
 
 // ---------------------------------------------------------------- solver --
@@ -1167,30 +1153,33 @@ void adjoint_horizon(cdns_ctx *c, const double *u0, const double *force, int nst
         CDNS_HIP(hipMemsetAsync(c->bc_prev, 0, (size_t)g.NQ * 2 * sizeof(zd), c->st));
         const int kc = hs.kc, nck = hs.nck;
         const size_t ckn = hs.ckn;
-        auto save = [&](int k) {
+        // the ten pieces of a checkpoint move in one launch: (u, u_prev, N_prev) planes and B_prev
+        auto checkpoint = [&](int k, bool restore) {
             zd *base = reinterpret_cast<zd *>(ck) + (size_t)k * ckn;
-            for (int i = 0; i < 3; ++i) {
-                CDNS_HIP(hipMemcpyAsync(base + (size_t)i * g.S, c->u[i], bplane, hipMemcpyDeviceToDevice, c->st));
-                CDNS_HIP(hipMemcpyAsync(base + (size_t)(3 + i) * g.S, c->up[i], bplane, hipMemcpyDeviceToDevice, c->st));
-                CDNS_HIP(hipMemcpyAsync(base + (size_t)(6 + i) * g.S, c->nlp[i], bplane, hipMemcpyDeviceToDevice, c->st));
+            CopyArgs a{};
+            for (int i = 0; i < 10; ++i) {
+                zd *state = i == 9 ? c->bc_prev : (i < 3 ? c->u[i] : (i < 6 ? c->up[i - 3] : c->nlp[i - 6]));
+                zd *kept = base + (size_t)i * g.S;
+                a.src[i] = restore ? kept : state;
+                a.dst[i] = restore ? state : kept;
+                a.n[i] = i == 9 ? (size_t)g.NQ * 2 : g.S;
             }
-            CDNS_HIP(hipMemcpyAsync(base + (size_t)9 * g.S, c->bc_prev, (size_t)g.NQ * 2 * sizeof(zd),
-                                    hipMemcpyDeviceToDevice, c->st));
+            a.count = 10;
+            Launch L(c, "checkpoint");
+            launch_copy_planes(a, c->st);
         };
-        auto restore = [&](int k) {
-            const zd *base = reinterpret_cast<const zd *>(ck) + (size_t)k * ckn;
-            for (int i = 0; i < 3; ++i) {
-                CDNS_HIP(hipMemcpyAsync(c->u[i], base + (size_t)i * g.S, bplane, hipMemcpyDeviceToDevice, c->st));
-                CDNS_HIP(hipMemcpyAsync(c->up[i], base + (size_t)(3 + i) * g.S, bplane, hipMemcpyDeviceToDevice, c->st));
-                CDNS_HIP(hipMemcpyAsync(c->nlp[i], base + (size_t)(6 + i) * g.S, bplane, hipMemcpyDeviceToDevice, c->st));
-            }
-            CDNS_HIP(hipMemcpyAsync(c->bc_prev, base + (size_t)9 * g.S, (size_t)g.NQ * 2 * sizeof(zd),
-                                    hipMemcpyDeviceToDevice, c->st));
-        };
+        // The forward pass leaves the last segment's synthesised fields in the segment storage, so
+        // that segment is neither checkpointed nor recomputed; and the last step of a recomputed
+        // segment ends with its synthesis.
+        const int last0 = (nck - 1) * kc + 1;
+        const size_t zstep = (size_t)6 * g.ZS * c->esz;
+        auto keep_synthesis = [&](int slot) { c->Zbuf = (char *)seg + (size_t)slot * zstep; };
         for (int it = 1; it <= nsteps; ++it) {
-            if ((it - 1) % kc == 0) save((it - 1) / kc);
+            if (it >= last0) keep_synthesis(it - last0);
+            else if ((it - 1) % kc == 0) checkpoint((it - 1) / kc, false);
             step(c, it);
         }
+        c->Zbuf = zkeep;
         // terminal objective and its gradient start the adjoint
         const double Jv = objective(c, objective_id, c->u, c->a_lu);
         if (J) *J = Jv;
@@ -1198,16 +1187,18 @@ void adjoint_horizon(cdns_ctx *c, const double *u0, const double *force, int nst
         zero_planes(c, c->a_lnp, 3, g.S);
         zero_planes(c, c->a_lf, 3, g.S);
         CDNS_HIP(hipMemsetAsync(c->a_lbp, 0, (size_t)g.NQ * 2 * sizeof(zd), c->st));
-        const size_t zstep = (size_t)6 * g.ZS * c->esz;
         for (int k = nck - 1; k >= 0; --k) {
             const int it0 = k * kc + 1, it1 = std::min((k + 1) * kc, nsteps);
-            restore(k);
-            // recompute the segment, keeping each step's synthesised (u, curl u)
-            for (int it = it0; it <= it1; ++it) {
-                c->Zbuf = (char *)seg + (size_t)(it - it0) * zstep;
-                step(c, it);
+            if (it0 != last0) {
+                checkpoint(k, true);
+                // recompute the segment, keeping each step's synthesised (u, curl u)
+                for (int it = it0; it <= it1; ++it) {
+                    keep_synthesis(it - it0);
+                    if (it < it1) step(c, it);
+                    else synthesise(c, c->u);
+                }
+                c->Zbuf = zkeep;
             }
-            c->Zbuf = zkeep;
             for (int it = it1; it >= it0; --it)
                 adjoint_step(c, it, (const char *)seg + (size_t)(it - it0) * zstep, force != nullptr);
         }
@@ -1667,7 +1658,9 @@ int cdns_cross_product(cdns_ctx *c, double *out, const double *av, const double 
         ref_to_planes(c, av, 3, 3, g.nj, a, where, g.JS);
         ref_to_planes(c, bv, 3, 3, g.nj, b, where, g.JS);
         zd *o[3] = {c->scr[0], c->scr[1], c->scr[2]};
-        cross_planes(c, a, b, o);
+        const zd *f6[6] = {a[0], a[1], a[2], b[0], b[1], b[2]};
+        backward_yz(c, f6, 6);
+        product_forward(c, o, nullptr, false);
         const zd *co[3] = {o[0], o[1], o[2]};
         planes_to_ref(c, co, 3, g.nj, out, 3, where, g.JS);
         if (where == CDNS_HOST) CDNS_HIP(hipStreamSynchronize(c->st));

@@ -125,6 +125,15 @@ void launch_real_planes_to_ref(const double *plane, double *ref, int nrow, int n
 void launch_widen(const void *src, zd *dst, size_t n, hipStream_t st);
 void launch_narrow(const zd *src, void *dst, size_t n, hipStream_t st);
 
+// plane copies in one launch
+struct CopyArgs {
+    const zd *src[10];
+    zd *dst[10];
+    size_t n[10];
+    int count;
+};
+void launch_copy_planes(const CopyArgs &a, hipStream_t st);
+
 struct CurlArgs {
     const zd *u[3];
     zd *w[3];
