@@ -769,7 +769,7 @@ void setup(cdns_ctx *c, double g_v) {
             for (int k = 0; k < 3; ++k) a.ctab_infl[i][k] = c->ctab[2 * k + i]; // PIr, VIv, VIf
         }
         Launch L(c, "setup_influence");
-        launch_solve(a, g.E, c->st);
+        launch_solve(a, c->st);
     }
     {
         Launch L(c, "setup_normalize");
@@ -783,14 +783,14 @@ void setup(cdns_ctx *c, double g_v) {
         a.sig_out = c->SIG0;
         for (int k = 0; k < 3; ++k) a.ctab_b[k] = c->ctab[6 + k]; // PBr, VBv, VBf
         Launch L(c, "setup_bproblem");
-        launch_solve(a, g.E, c->st);
+        launch_solve(a, c->st);
     }
     c->pa = c->cfg.a_pre0;
     c->pb = c->cfg.b_pre0;
     {
         Launch L(c, "setup_pg_response");
         launch_pg_response(c->WAVX, c->WAVZ, c->WL, c->WD, c->WR, c->ad_v, g_v, c->cfg.Re, c->cfg.a_V, c->cfg.b_V,
-                           g.NYS, g.JS, g.NZS, c->u_unit, c->w_unit, c->q_unit, g.E, c->st);
+                           g.NYS, g.JS, g.NZS, c->u_unit, c->w_unit, c->q_unit, c->st);
     }
     c->setup_done = true;
 }
@@ -840,7 +840,7 @@ void step(cdns_ctx *c, int it) {
     a.sigma = 1;
     {
         Launch L(c, "solve_step");
-        launch_solve(a, c->g.E, c->st);
+        launch_solve(a, c->st);
     }
     for (int k = 0; k < 3; ++k) {
         std::swap(c->u[k], c->up[k]);
@@ -1733,7 +1733,7 @@ int cdns_solve_modes(cdns_ctx *c, double *pressure, const double *rhs_p, const d
         // column before it writes it.
         {
             Launch L(c, "solve_modes");
-            launch_solve(a, g.E, c->st);
+            launch_solve(a, c->st);
         }
         const zd *cp[1] = {c->scr[4]};
         planes_to_ref(c, cp, 1, g.nj, pressure, 1, where, g.JS);

@@ -234,7 +234,7 @@ void launch_planes_finite(const zd *const *planes, int n, int NQ, int JS, int ny
                           hipStream_t st);
 void launch_plane_moments(const DiagArgs &a, hipStream_t st);
 
-void launch_solve(const SolveArgs &a, int E, hipStream_t st);
+void launch_solve(const SolveArgs &a, hipStream_t st);
 // ad and wn tables of the pressure (0) and the velocity (1) operator
 struct AdArgs {
     const double *WAVX, *WAVZ, *WL, *WD, *WR;
@@ -247,6 +247,6 @@ void launch_normalize_influence(zd *ID0, zd *ID1, int NQ, int root_q, double aV1
 void launch_pg_response(const double *WAVX, const double *WAVZ, const double *WL, const double *WD,
                         const double *WR, const double *ad_v, double g_v, double Re, const double *aV,
                         const double *bV, int ny, int JS, int root_q, double *u_unit, double *w_unit,
-                        double *q_unit, int E, hipStream_t st);
+                        double *q_unit, hipStream_t st);
 
 } // namespace cdns

@@ -144,7 +144,7 @@ __device__ inline void store_compact(double *const (&t)[3], size_t off, int lane
 // (simulation.cpp:111-140) fused in MODE_STEP; the setup problems of eqsolve_pv.cpp:266-303
 // and 452-477 in MODE_INFLUENCE / MODE_BPROBLEM.
 template <int NE, int MODE, bool NL32 = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE == 2 ? 3 : 1))) k_solve(SolveArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE <= 3 ? 5 - NE : 1))) k_solve(SolveArgs a) {
     const int lane = lane_id(), p = sp::parity(lane);
     // the column index is wavefront-uniform: made visible as such, the per-column scalars
     // (wavenumbers, wall values, influence and sigma entries) come through scalar loads.
@@ -499,12 +499,19 @@ template <int NE> static void launch_solve_mode(const SolveArgs &a, hipStream_t 
     default: throw std::runtime_error("unknown solve mode");
     }
 }
-// E = column stride / 64 complex entries per lane pair: two entries of one chain per lane for
-// columns up to 128, four up to 256
-void launch_solve(const SolveArgs &a, int E, hipStream_t st) {
-    if (E == 2) launch_solve_mode<2>(a, st);
-    else if (E == 4) launch_solve_mode<4>(a, st);
-    else throw std::runtime_error("unsupported column length");
+// NE entries of one chain per lane: the smallest that holds the column, so that no lane group is idle and the
+// registers follow the length (the step's solve 102, 168, 223 and 286 VGPRs: 4, 3, 2 and 1 wavefronts per SIMD
+// asked of the compiler, which is what bounds the long columns).  us per launch with 2 entries up to 128 and
+// 4 beyond, and so: 31-entry columns of 32 x 33 x 32 13.1 / 11.8 (both of those are mostly the launch and one
+// wavefront's dependent scans), 63 of 64 x 65 x 64 22.2 / 20.3, 191 of 256 x 193 x 192, mixed 509.9 / 316.6
+void launch_solve(const SolveArgs &a, hipStream_t st) {
+    switch (a.ny / 64 + 1) {
+    case 1: launch_solve_mode<1>(a, st); break;
+    case 2: launch_solve_mode<2>(a, st); break;
+    case 3: launch_solve_mode<3>(a, st); break;
+    case 4: launch_solve_mode<4>(a, st); break;
+    default: throw std::runtime_error("unsupported column length");
+    }
 }
 
 // build_wn_ad (eqsolve_pv.cpp:148-168) for the pressure and the velocity operator: a continued-fraction
@@ -614,13 +621,18 @@ __global__ void k_pg_response(const double *WAVX, const double *WAVZ, const doub
 }
 void launch_pg_response(const double *WAVX, const double *WAVZ, const double *WL, const double *WD, const double *WR,
                         const double *ad_v, double g_v, double Re, const double *aV, const double *bV, int ny, int JS,
-                        int root_q, double *u_unit, double *w_unit, double *q_unit, int E, hipStream_t st) {
-    if (E == 2)
-        hipLaunchKernelGGL((k_pg_response<2>), dim3(1), dim3(64), 0, st, WAVX, WAVZ, WL, WD, WR, ad_v, g_v, Re, aV[0],
-                           bV[0], aV[2], bV[2], ny, JS, root_q, u_unit, w_unit, q_unit);
-    else
-        hipLaunchKernelGGL((k_pg_response<4>), dim3(1), dim3(64), 0, st, WAVX, WAVZ, WL, WD, WR, ad_v, g_v, Re, aV[0],
-                           bV[0], aV[2], bV[2], ny, JS, root_q, u_unit, w_unit, q_unit);
+                        int root_q, double *u_unit, double *w_unit, double *q_unit, hipStream_t st) {
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(64), 0, st, WAVX, WAVZ, WL, WD, WR, ad_v, g_v, Re, aV[0], bV[0],
+                           aV[2], bV[2], ny, JS, root_q, u_unit, w_unit, q_unit);
+    };
+    switch (ny / 64 + 1) {
+    case 1: go(k_pg_response<1>); break;
+    case 2: go(k_pg_response<2>); break;
+    case 3: go(k_pg_response<3>); break;
+    case 4: go(k_pg_response<4>); break;
+    default: throw std::runtime_error("unsupported column length");
+    }
 }
 
 } // namespace cdns
