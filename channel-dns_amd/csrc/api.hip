@@ -806,8 +806,9 @@ void step_coefficients(int it, double dt, double Re, double co[5]) {
     co[4] = (a0 + a1) * Re;
 }
 
-// One iteration of Simulation::run (simulation.cpp:173-191) with enqueue_serial_step (142-171).
-void step(cdns_ctx *c, int it) {
+// One iteration of Simulation::run (simulation.cpp:173-191) with enqueue_serial_step (142-171).  The next
+// step does not read the pressure, so a step that another follows inside one call does not write it.
+void step(cdns_ctx *c, int it, bool pressure = true) {
     double co[5];
     step_coefficients(it, c->cfg.DT, c->cfg.Re, co);
     if (it < 3) {
@@ -835,7 +836,7 @@ void step(cdns_ctx *c, int it) {
     a.bcw = c->bcw;
     a.bc_prev = c->bc_prev;
     a.bc_ext = c->bc_ext;
-    a.P = c->P_;
+    a.P = pressure ? c->P_ : nullptr;
     a.correct = 1;
     a.sigma = 1;
     {
@@ -1177,7 +1178,7 @@ void adjoint_horizon(cdns_ctx *c, const double *u0, const double *force, int nst
         for (int it = 1; it <= nsteps; ++it) {
             if (it >= last0) keep_synthesis(it - last0);
             else if ((it - 1) % kc == 0) checkpoint((it - 1) / kc, false);
-            step(c, it);
+            step(c, it, it == nsteps);
         }
         c->Zbuf = zkeep;
         // terminal objective and its gradient start the adjoint
@@ -1194,7 +1195,7 @@ void adjoint_horizon(cdns_ctx *c, const double *u0, const double *force, int nst
                 // recompute the segment, keeping each step's synthesised (u, curl u)
                 for (int it = it0; it <= it1; ++it) {
                     keep_synthesis(it - it0);
-                    if (it < it1) step(c, it);
+                    if (it < it1) step(c, it, false);
                     else synthesise(c, c->u);
                 }
                 c->Zbuf = zkeep;
@@ -1845,7 +1846,7 @@ int cdns_step(cdns_ctx *c, int it) {
 
 int cdns_run(cdns_ctx *c, int it_begin, int nsteps) {
     try {
-        for (int i = 0; i < nsteps; ++i) step(c, it_begin + i);
+        for (int i = 0; i < nsteps; ++i) step(c, it_begin + i, i == nsteps - 1);
         return 0;
     } catch (const std::exception &e) {
         return fail(c, e);

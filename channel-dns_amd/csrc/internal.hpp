@@ -178,7 +178,7 @@ struct SolveArgs {
     const double *q_unit;
     double grad_x, grad_z, qx_mean, qz_mean;
     int grad_pre;
-    // outputs
+    // outputs (step: P may be null, a pressure that is not asked for)
     zd *P, *V[3];
     // influence, per wall: pressure, velocity, raw wall divergence [q][2], compact tables (P, v, phi)
     zd *infl_P[2], *infl_V[2][3], *infl_div[2];

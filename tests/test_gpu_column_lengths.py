@@ -28,3 +28,20 @@ def test_step_at_column_length(gpu, nj):
         print(f"{nj} entries, {name}: {err:.2e}")
         assert np.isfinite(got).all() and err < 1e-10
     dev.close()
+
+
+@pytest.mark.parametrize("compact", [True, False])
+def test_pressure_of_a_run_is_that_of_single_steps(gpu, compact):
+    """A run writes only its last step's pressure; every step of it writes the rest of the state.  Both table
+    forms (u and w with wall conditions of their own have no compact one)."""
+    cfg = config.make(16, 34, 16, 6, 30, 6, 20, 48, 18, 4 * math.pi, 2 * math.pi, 180.0, 1e-4,
+                      **({} if compact else {"a_V": (1.0, 1.0, 0.5), "b_V": (0.0, 0.0, 0.1)}))
+    u0 = fields.seeded_velocity(cfg, seed=7)
+    run, steps = gpu.Channel(cfg), gpu.Channel(cfg)
+    for dev in (run, steps):
+        dev.set_state("velocity", u0)
+    run.run(4, it_begin=1)
+    for it in range(1, 5):
+        steps.step(it)
+    for name in ("velocity", "pressure"):
+        assert np.array_equal(run.get_state(name), steps.get_state(name))
