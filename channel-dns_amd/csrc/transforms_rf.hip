@@ -39,9 +39,6 @@ __device__ inline cpx<R> herm_pack(const cpx<R> *A, const cpx<R> *B, int k, int 
     return {av.x - bv.y, av.y + bv.x};
 }
 
-// herm_pack without branches: both loads are issued for every lane (index clamped to the
-// retained range) and the value is selected afterwards, so a wavefront's loads of several lines
-// can all be in flight at once.
 // Element `row + i` of a field given by its kernel-argument base: a 32-bit byte offset from a
 // wavefront-uniform base, so the load takes the scalar-base addressing form.
 template <typename T> __device__ inline T ld_row(const T *base, unsigned row, int i) {
@@ -49,16 +46,42 @@ template <typename T> __device__ inline T ld_row(const T *base, unsigned row, in
     return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
 }
 
-template <typename R>
-__device__ inline cpx<R> herm_pack_nb(const cpx<R> *A, const cpx<R> *B, unsigned row, int k, int N, int K, bool use) {
-    const bool mirror = k > K, zero = !use || (mirror && N - k > K);
-    int src = mirror ? N - k : k;
-    src = src < 0 ? 0 : (src > K ? K : src);
-    const cpx<R> av = ld_row(A, row, src), bv = ld_row(B, row, src);
-    const bool real_end = src == 0 || 2 * src == N;
-    const R ay = real_end ? R(0) : (mirror ? -av.y : av.y), by = real_end ? R(0) : (mirror ? -bv.y : bv.y);
-    return zero ? cpx<R>{R(0), R(0)} : cpx<R>{av.x - by, ay + bv.x};
-}
+// Hermitian packing of the slots k = lo + d, 0 <= d < D (d this lane's, lo and D compile-time), whose rule is
+// mostly the same for all of them: retained as they are (k <= K), conjugates of slot N - k, or zero.  The
+// wavefront then decides once, in scalar registers, and a slot costs an index and two additions; only slots
+// that straddle a limit (or hold the real DC and Nyquist coefficients) are decided lane by lane.  The FP32 x
+// product is bound by vector-ALU issue, of which the selects of every slot were an eighth: 196 x 193 x 196 67.4 ->
+// 63.9 us, 384 x 289 x 288 507 -> 467; FP64 96 x 97 x 96 (132 -> 116 VGPRs) 23.7 -> 23.3.
+template <int N, int LO, int D, bool U> struct HermSlots {
+    // 0 lane by lane, 1 direct, 2 mirrored, 3 zero
+    static __device__ inline int kind(int K) {
+        constexpr int HI = LO + D - 1;
+        if (!U || LO == 0) return 0;
+        if (HI <= K && !(2 * K == N && LO <= N / 2 && HI >= N / 2)) return 1;
+        if (LO > K && LO >= N - K) return 2;
+        if (LO > K && HI < N - K) return 3;
+        return 0;
+    }
+    static __device__ inline int source(int kind, int d, int K) {
+        if (kind == 0) {
+            const int k = LO + d, src = k > K ? N - k : k;
+            return src > K ? K : src;
+        }
+        const int c = kind == 1 ? LO : (kind == 2 ? N - LO : 0), sg = kind == 1 ? 1 : (kind == 2 ? -1 : 0);
+        return c + sg * d;
+    }
+    template <typename R> static __device__ inline cpx<R> value(int kind, int d, int K, cpx<R> av, cpx<R> bv) {
+        if (kind == 0) {
+            const int k = LO + d;
+            const bool mirror = k > K, zero = mirror && N - k > K, real_end = k == 0 || 2 * k == N;
+            const R ay = real_end ? R(0) : (mirror ? -av.y : av.y), by = real_end ? R(0) : (mirror ? -bv.y : bv.y);
+            return zero ? cpx<R>{R(0), R(0)} : cpx<R>{av.x - by, ay + bv.x};
+        }
+        if (kind == 3) return {R(0), R(0)};
+        const R sg = kind == 1 ? R(1) : R(-1);
+        return {av.x - sg * bv.y, bv.x + sg * av.y};
+    }
+};
 
 template <typename R, int N>
 __device__ inline void load_roots(cpx<R> *tw, const void *src) {
@@ -179,15 +202,30 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
     // the first transform costs some 50 more VGPRs in FP64
     cpx<R> ph[3][MH];
     const unsigned prow = (unsigned)(valid ? p : 0) * (unsigned)a.nkx;
+    // slots 2 N1 m + d of this lane (lanes past the rows repeat the last one; a point past the end repeats
+    // point 0; neither is used)
+    const int d = (t < N1 ? t : N1 - 1) + N1 * h;
+    // FP64 rows of 14 points and more are bound by latency at 2 or 3 wavefronts per SIMD, where the branches cost
+    // more than the selects they replace (196-point lines 107 us without, 110 with)
+    constexpr bool kUniform = sizeof(R) == 4 || MH <= 6;
     auto load_line = [&](auto line) {
         constexpr int LN = decltype(line)::value;
         const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN]);
         const cpx<R> *Bv = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN + 1]);
+        cpx<R> av[H2], bv[H2];
+        sfor<0, H2>([&](auto m) {
+            constexpr int M = decltype(m)::value;
+            using HS = HermSlots<N, 2 * N1 * M, 2 * N1, kUniform>;
+            const int src = HS::source(HS::kind(K), d, K);
+            av[M] = ld_row(A, prow, src);
+            bv[M] = ld_row(Bv, prow, src);
+        });
         sfor<0, MH>([&](auto m) {
             constexpr int M = decltype(m)::value;
-            if constexpr (M < H2)
-                ph[LN][M] = herm_pack_nb(A, Bv, prow, t + N1 * (2 * M + h), N, K, valid && t < N1);
-            else
+            if constexpr (M < H2) {
+                using HS = HermSlots<N, 2 * N1 * M, 2 * N1, kUniform>;
+                ph[LN][M] = HS::template value<R>(HS::kind(K), d, K, av[M], bv[M]);
+            } else
                 ph[LN][M] = cpx<R>{R(0), R(0)};
         });
     };
