@@ -80,9 +80,10 @@ struct XArgs {
     int coarse; // coarse-grid transform: at NXS = N/2 the Nyquist coefficient counts twice
     double *phys; // reference-layout physical field(s) for the single-field stages
     size_t phys_fs; // x backward of several fields: stride of the physical fields
-    // product a x b: input fields a0 a1 a2 b0 b1 b2 and the three output fields
-    const void *fin[6];
-    void *fout[3];
+    // products a x b (blockIdx.y): input fields a0 a1 a2 b0 b1 b2 and the three output fields
+    const void *fin[2][6];
+    void *fout[2][3];
+    int nprod;
 };
 
 void launch_ybwd(const YArgs &a, int nfields, bool fp32, hipStream_t st);

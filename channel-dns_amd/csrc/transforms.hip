@@ -271,8 +271,8 @@ __global__ void __launch_bounds__(256) k_xprod(XArgs a) {
         const int pt = p0 + pp;
         cpx<R> v = {R(0), R(0)};
         if (pt < np) {
-            const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[2 * gsel]) + (size_t)pt * a.nkx;
-            const cpx<R> *B = reinterpret_cast<const cpx<R> *>(a.fin[2 * gsel + 1]) + (size_t)pt * a.nkx;
+            const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * gsel]) + (size_t)pt * a.nkx;
+            const cpx<R> *B = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * gsel + 1]) + (size_t)pt * a.nkx;
             v = pack_c2r(A, B, k, N, K);
         }
         buf[e] = v;
@@ -330,8 +330,8 @@ __global__ void __launch_bounds__(256) k_xprod(XArgs a) {
         if (sel < 2) { pa = pb = 2 * h + sel; ca = 0; cb = 1; }
         else { pa = 2 * h; pb = 2 * h + 1; ca = cb = 2; }
         const int pta = p0 + pa, ptb = p0 + pb;
-        if (pta < np) reinterpret_cast<cpx<R> *>(a.fout[ca])[zline_index(pta, k, a.nkx, a.NZ2)] = first;
-        if (ptb < np) reinterpret_cast<cpx<R> *>(a.fout[cb])[zline_index(ptb, k, a.nkx, a.NZ2)] = second;
+        if (pta < np) reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][ca])[zline_index(pta, k, a.nkx, a.NZ2)] = first;
+        if (ptb < np) reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][cb])[zline_index(ptb, k, a.nkx, a.NZ2)] = second;
     }
 }
 
@@ -477,7 +477,7 @@ void launch_xprod(const XArgs &a, bool fp32, hipStream_t st) {
     if (a.rf && (launch_xprod_rf(a, fp32, st) || launch_xprod_line(a, fp32, st))) return;
     const int it = items_per_thread(3 * a.P, a.plan);
     if ((a.P / 2) * a.plan.n > 8 * 256) throw std::runtime_error("x-product batch too large");
-    dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P);
+    dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P, a.nprod);
     if (fp32) {
         const size_t sm = (size_t)3 * a.P * a.plan.n * sizeof(cpx<float>);
         CDNS_DISPATCH_IT(k_xprod, float, it, grid, sm, st, a);

@@ -20,8 +20,8 @@ __global__ void __launch_bounds__(512) k_xprod_line(XArgs a, LinePlan p) {
     const bool on = lane_on && j < P;
     const bool valid = on && p0 + j < np;
     {
-        const void *fa = i == 0 ? a.fin[0] : (i == 1 ? a.fin[2] : a.fin[4]);
-        const void *fb = i == 0 ? a.fin[1] : (i == 1 ? a.fin[3] : a.fin[5]);
+        const void *fa = i == 0 ? a.fin[blockIdx.y][0] : (i == 1 ? a.fin[blockIdx.y][2] : a.fin[blockIdx.y][4]);
+        const void *fb = i == 0 ? a.fin[blockIdx.y][1] : (i == 1 ? a.fin[blockIdx.y][3] : a.fin[blockIdx.y][5]);
         const size_t row = (size_t)(valid ? p0 + j : 0) * a.nkx;
         const cpx<R> *A = reinterpret_cast<const cpx<R> *>(fa) + row, *B = reinterpret_cast<const cpx<R> *>(fb) + row;
         load_line_roots<R>(tw, a.tw, N);
@@ -54,8 +54,8 @@ __global__ void __launch_bounds__(512) k_xprod_line(XArgs a, LinePlan p) {
     if (pw >= np) return;
     const int wl = pw / a.NZ2;
     const size_t base = ((size_t)wl * a.nkx) * a.NZ2 + (pw - wl * a.NZ2);
-    cpx<R> *o0 = reinterpret_cast<cpx<R> *>(a.fout[0]) + base, *o1 = reinterpret_cast<cpx<R> *>(a.fout[1]) + base,
-           *o2 = reinterpret_cast<cpx<R> *>(a.fout[2]) + base;
+    cpx<R> *o0 = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][0]) + base, *o1 = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][1]) + base,
+           *o2 = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][2]) + base;
     const cpx<R> *F = buf + 3 * wj * lb, *Z = buf + (3 * (wj & ~1) + 1) * lb;
     for (int k = threadIdx.x / P; k < a.nkx; k += blockDim.x / P) {
         const int m = k == 0 ? 0 : N - k;
@@ -79,7 +79,7 @@ template <typename R, bool BIG> void go_xprod_line(XArgs a, const LinePlan &p, h
     const size_t lds = ((size_t)3 * P * p.lb + p.n) * sizeof(cpx<R>);
     a.P = P;
     allow_lds(k_xprod_line<R, BIG>, lds);
-    hipLaunchKernelGGL((k_xprod_line<R, BIG>), dim3((a.NL * a.NZ2 + P - 1) / P), dim3(64 * waves), lds, st, a, p);
+    hipLaunchKernelGGL((k_xprod_line<R, BIG>), dim3((a.NL * a.NZ2 + P - 1) / P, a.nprod), dim3(64 * waves), lds, st, a, p);
 }
 } // namespace
 

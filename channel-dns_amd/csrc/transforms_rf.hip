@@ -107,8 +107,8 @@ __global__ void __launch_bounds__(64) k_xprod_rf(XArgs a) {
     sfor<0, 3>([&](auto line) {
         constexpr int LN = decltype(line)::value;
         cpx<R> x[MX];
-        const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN]) + (size_t)p * a.nkx;
-        const cpx<R> *Bv = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN + 1]) + (size_t)p * a.nkx;
+        const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * LN]) + (size_t)p * a.nkx;
+        const cpx<R> *Bv = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * LN + 1]) + (size_t)p * a.nkx;
         sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
         if (valid && t < N1) sfor<0, N2>([&](auto n2) { x[n2] = herm_pack(A, Bv, t + N1 * decltype(n2)::value, N, K); });
         two_pass<R, N1, N2, +1>(x, t, tw, B, wsync);
@@ -129,8 +129,8 @@ __global__ void __launch_bounds__(64) k_xprod_rf(XArgs a) {
         });
     }
     const R half = R(0.5) / R(N);
-    cpx<R> *Nx = reinterpret_cast<cpx<R> *>(a.fout[0]), *Ny = reinterpret_cast<cpx<R> *>(a.fout[1]),
-           *Nz = reinterpret_cast<cpx<R> *>(a.fout[2]);
+    cpx<R> *Nx = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][0]), *Ny = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][1]),
+           *Nz = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][2]);
     // forward of (Nx + i Ny): transposed plan, input already in place
     two_pass<R, N2, N1, -1>(F, t, tw, B, wsync);
     if (t < N1) sfor<0, N2>([&](auto k1) { B[t + N1 * decltype(k1)::value] = F[k1]; });
@@ -210,8 +210,8 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
     constexpr bool kUniform = sizeof(R) == 4 || MH <= 6;
     auto load_line = [&](auto line) {
         constexpr int LN = decltype(line)::value;
-        const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN]);
-        const cpx<R> *Bv = reinterpret_cast<const cpx<R> *>(a.fin[2 * LN + 1]);
+        const cpx<R> *A = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * LN]);
+        const cpx<R> *Bv = reinterpret_cast<const cpx<R> *>(a.fin[blockIdx.y][2 * LN + 1]);
         cpx<R> av[H2], bv[H2];
         sfor<0, H2>([&](auto m) {
             constexpr int M = decltype(m)::value;
@@ -305,7 +305,7 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
         const int wl = pw / a.NZ2;
         const size_t wbase = ((size_t)wl * a.nkx) * a.NZ2 + (pw - wl * a.NZ2);
         for (int fo = 0; fo < 3; ++fo) {
-            cpx<R> *out = reinterpret_cast<cpx<R> *>(a.fout[fo]) + wbase;
+            cpx<R> *out = reinterpret_cast<cpx<R> *>(a.fout[blockIdx.y][fo]) + wbase;
             for (int k = wr; k < a.nkx; k += 64 * W / PB) out[(size_t)k * a.NZ2] = buf[wj][fo * a.nkx + k];
         }
     }
@@ -502,13 +502,14 @@ template <typename R, int N1, int N2> static void go_xprod(const XArgs &a, hipSt
         // the three retained rows of a point are staged in its transpose buffer
         if (a.pair && 3 * a.nkx <= 2 * xbuf_entries<N1, N2>()) {
             constexpr int PB = kXWaves<R> * PGeo<N1, N2>::NG;
-            hipLaunchKernelGGL((k_xprod_pair<R, N1, N2>), dim3((a.NL * a.NZ2 + PB - 1) / PB), dim3(64 * kXWaves<R>),
-                               0, st, a);
+            hipLaunchKernelGGL((k_xprod_pair<R, N1, N2>), dim3((a.NL * a.NZ2 + PB - 1) / PB, a.nprod),
+                               dim3(64 * kXWaves<R>), 0, st, a);
             return;
         }
     }
     using Gm = Geo<N1, N2>;
-    hipLaunchKernelGGL((k_xprod_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + Gm::NG - 1) / Gm::NG), dim3(64), 0, st, a);
+    hipLaunchKernelGGL((k_xprod_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + Gm::NG - 1) / Gm::NG, a.nprod), dim3(64), 0,
+                       st, a);
 }
 template <typename R, int N1, int N2> static void go_zbwd(const ZArgs &a, int nf, hipStream_t st) {
     if constexpr (N1 % 2 == 0 && N2 % 2 == 0) {
