@@ -251,4 +251,14 @@ __device__ inline int xcd_block(int nblocks) {
     return xcd < tall ? xcd * per + local : tall * per + (xcd - tall) * (per - 1) + local;
 }
 
+// The same in runs of `run` logical blocks per XCD, dealt out in turn: the XCDs then work side by side in
+// one neighbourhood of memory.  The last nblocks mod (8 run) blocks keep their order.
+__device__ inline int xcd_run(int nblocks, int run) {
+    constexpr int X = 8;
+    const int b = blockIdx.x, turn = X * run;
+    if (b >= nblocks - nblocks % turn) return b;
+    const int k = b / X, t = k / run;
+    return t * turn + (b % X) * run + (k - t * run);
+}
+
 } // namespace cdns

@@ -13,7 +13,7 @@ __global__ void __launch_bounds__(512) k_xprod_line(XArgs a, LinePlan p) {
     cpx<R> *tw = reinterpret_cast<cpx<R> *>(smem_raw), *buf = tw + p.n;
     const int N = p.n, K = a.nkx - 1, P = a.P, lb = p.lb;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / p.gs, t = lane - g * p.gs;
-    const int np = a.NL * a.NZ2, p0 = blockIdx.x * P;
+    const int np = a.NL * a.NZ2, p0 = xcd_block((int)gridDim.x) * P;
     const int line = wv * p.ng + g; // backward: line i of point j at 3 j + i
     const bool lane_on = g < p.ng;
     const int j = line / 3, i = line - 3 * j;

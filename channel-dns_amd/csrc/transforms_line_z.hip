@@ -13,7 +13,8 @@ __global__ void __launch_bounds__(512) k_zbwd_line(ZArgs a, LinePlan p) {
     const int N = p.n, NZS = a.NZS, KT = a.KT;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / p.gs, t = lane - g * p.gs;
     const int line = wv * p.ng + g;
-    const int kx0 = blockIdx.x * KT, l = blockIdx.y, f = blockIdx.z;
+    const int nb = (a.nkx + KT - 1) / KT, L = xcd_block((int)gridDim.x);
+    const int lf = L / nb, kx0 = (L - lf * nb) * KT, f = lf / a.NL, l = lf - f * a.NL;
     const int nl = min(KT, a.nkx - kx0);
     const bool on = g < p.ng && line < nl;
     const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.NQ +
@@ -83,7 +84,7 @@ template <typename R, bool BIG> void go_zbwd_line(ZArgs a, const LinePlan &p, in
     const int nb = (a.nkx + cap - 1) / cap;
     a.KT = (a.nkx + nb - 1) / nb;
     allow_lds(k_zbwd_line<R, BIG>, lds(a.KT));
-    hipLaunchKernelGGL((k_zbwd_line<R, BIG>), dim3((a.nkx + a.KT - 1) / a.KT, a.NL, nf), dim3(64 * waves(a.KT)),
+    hipLaunchKernelGGL((k_zbwd_line<R, BIG>), dim3((a.nkx + a.KT - 1) / a.KT * a.NL * nf), dim3(64 * waves(a.KT)),
                        lds(a.KT), st, a, p);
 }
 template <typename R, bool BIG> void go_zfwd_line(ZArgs a, const LinePlan &p, int nf, hipStream_t st) {

@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(64) k_xprod_rf(XArgs a) {
     load_roots<R, N>(tw, a.tw);
     __syncthreads();
     const int np = a.NL * a.NZ2, K = a.nkx - 1;
-    const int p = blockIdx.x * NG + g;
+    const int p = xcd_run((int)gridDim.x, kXRun / NG) * NG + g;
     const bool valid = p < np;
     cpx<R> *B = buf[g];
     cpx<R> ph[3][MX];
@@ -194,7 +194,7 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / G, r = lane - g * G, t = r >> 1, h = r & 1;
     const int gb = wv * NG + g;
     const int np = a.NL * a.NZ2, K = a.nkx - 1;
-    const int p0 = blockIdx.x * PB, p = p0 + gb;
+    const int p0 = xcd_run((int)gridDim.x, kXRun / PB) * PB, p = p0 + gb;
     const bool valid = p < np;
     cpx<R> *B0 = buf[gb], *B1 = buf[gb] + XB;
     // each line's loads are branch-free, so they are all in flight before the first use; the
@@ -368,7 +368,8 @@ __global__ void __launch_bounds__((kZThreads<R, N1, N2>)) k_zbwd_rf(ZArgs a) {
     const int line = wv * NG + g;
     load_roots<R, N>(tw, a.tw);
     __syncthreads();
-    const int kx0 = blockIdx.x * kZLines, kx = kx0 + line, l = blockIdx.y, f = blockIdx.z;
+    const int nb = (a.nkx + kZLines - 1) / kZLines, L = xcd_run((int)gridDim.x, kZRun * nb);
+    const int lf = L / nb, kx0 = (L - lf * nb) * kZLines, kx = kx0 + line, f = lf / a.NL, l = lf - f * a.NL;
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
@@ -408,7 +409,7 @@ __global__ void __launch_bounds__(64) k_zfwd_rf(ZArgs a) {
     __shared__ cpx<R> buf[NG][LB];
     const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
     // neighbouring kx groups of one (field, l) read the same cache lines: keep them on one XCD
-    const int L = xcd_block((int)gridDim.x);
+    const int L = xcd_run((int)gridDim.x, kZRun * a.nkxg);
     const int kxg = L % a.nkxg, lf = L / a.nkxg, l = lf % a.NL, f = lf / a.NL;
     const int kx = kxg * NG + g;
     const bool valid = kx < a.nkx;
@@ -461,7 +462,8 @@ __global__ void __launch_bounds__((kZPThreads<R, N1, N2>)) k_zbwd_pair(ZArgs a) 
     __shared__ cpx<R> lds[T::LDS];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / G, r = lane - g * G, t = r >> 1, h = r & 1;
     const int line = wv * NG + g;
-    const int kx0 = blockIdx.x * kZLines, kx = kx0 + line, l = blockIdx.y, f = blockIdx.z;
+    const int nb = (a.nkx + kZLines - 1) / kZLines, L = xcd_run((int)gridDim.x, kZRun * nb);
+    const int lf = L / nb, kx0 = (L - lf * nb) * kZLines, kx = kx0 + line, f = lf / a.NL, l = lf - f * a.NL;
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
@@ -515,13 +517,13 @@ template <typename R, int N1, int N2> static void go_zbwd(const ZArgs &a, int nf
     if constexpr (N1 % 2 == 0 && N2 % 2 == 0) {
         if (a.pair) {
             using T = ZTileP<R, N1, N2>;
-            hipLaunchKernelGGL((k_zbwd_pair<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB, a.NL, nf),
+            hipLaunchKernelGGL((k_zbwd_pair<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB * a.NL * nf),
                                dim3(64 * T::WAVES), 0, st, a);
             return;
         }
     }
     using T = ZTile<R, N1, N2>;
-    hipLaunchKernelGGL((k_zbwd_rf<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB, a.NL, nf), dim3(64 * T::WAVES), 0,
+    hipLaunchKernelGGL((k_zbwd_rf<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB * a.NL * nf), dim3(64 * T::WAVES), 0,
                        st, a);
 }
 template <typename R, int N1, int N2> static void go_zfwd(const ZArgs &a, int nf, hipStream_t st) {
