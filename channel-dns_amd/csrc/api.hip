@@ -303,6 +303,7 @@ YArgs yargs(cdns_ctx *c) {
     a.njo = g.nj / 2;
     a.JS = g.JS;
     a.NQ = g.NQ;
+    a.QP = g.QP;
     a.NLH = g.NLH;
     a.NY2 = g.NY2;
     a.YS = g.YS;
@@ -322,6 +323,7 @@ DctArgs dct_args(cdns_ctx *c) {
     a.ny = g.NYS;
     a.JS = g.JS;
     a.NQ = g.NQ;
+    a.QP = g.QP;
     a.nzk = g.nzk;
     a.NY2 = g.NY2;
     a.L = 2 * g.NY2;
@@ -339,7 +341,7 @@ ZArgs zargs(cdns_ctx *c, const void *in, void *out, size_t in_fs, size_t out_fs)
     a.nkx = c->g.nkx;
     a.nzk = c->g.nzk;
     a.NZS = c->g.NZS;
-    a.NQ = c->g.NQ;
+    a.QP = c->g.QP;
     a.KT = c->KT;
     a.NL = c->g.NL;
     a.rf = c->rf;
@@ -479,13 +481,13 @@ YArgs yargs_coarse(cdns_ctx *c) {
     a.coef = c->cy_b;
     a.NLH = c->g.NY / 2 + 1;
     a.NY2 = c->g.NY;
-    a.YS = (size_t)(c->g.NY + 1) * c->g.NQ;
+    a.YS = (size_t)(c->g.NY + 1) * c->g.QP;
     return a;
 }
 size_t coarse_points(const cdns_ctx *c) { return (size_t)c->g.NZ * (c->g.NY + 1) * c->g.NX; }
 size_t coarse_zs(const cdns_ctx *c) { return (size_t)(c->g.NY + 1) * c->g.NZ * c->g.nkx; }
 ZArgs zargs_coarse(cdns_ctx *c, const void *in, void *out) {
-    const size_t ys = (size_t)(c->g.NY + 1) * c->g.NQ;
+    const size_t ys = (size_t)(c->g.NY + 1) * c->g.QP;
     ZArgs a = zargs(c, in, out, ys, coarse_zs(c));
     a.tw = c->ctwz;
     a.plan = c->cpz;
@@ -1262,7 +1264,12 @@ int cdns_create(const cdns_config *cfg, cdns_ctx **out) {
         g.NL = g.NY2 + 1;
         g.NLH = g.NY2 / 2 + 1;
         g.S = (size_t)g.NQ * g.JS;
-        g.YS = (size_t)g.NL * g.NQ;
+        // rows of whole cache lines in both precisions, so that the y stages' 8-column segments are whole lines
+        // (or halves) too.  us per launch against rows of NQ, y backward with the curl / y forward: 384 x 289 x
+        // 288 FP32 245 / 114 -> 237 / 108, 196 x 193 x 196 FP32 45.4 / 27.2 -> 43.2 / 27.1, FP64 71.1 / 39.8 ->
+        // 70.2 / 39.7
+        g.QP = (g.NQ + 15) / 16 * 16;
+        g.YS = (size_t)g.NL * g.QP;
         g.ZS = (size_t)g.NL * g.NZ2 * g.nkx;
         CDNS_HIP(hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking));
         CDNS_HIP(hipGetDevice(&c->device));

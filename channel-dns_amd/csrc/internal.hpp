@@ -12,7 +12,7 @@ struct YArgs {
     const zd *add[6];  // yfwd: planes added to the outputs (a body force), or null
     void *y;           // Y fields, field f at y + f*YS (element type by precision)
     const double *coef, *coef2;
-    int nj, nje, njo, JS, NQ, NLH, NY2, nwj, ng;
+    int nj, nje, njo, JS, NQ, QP, NLH, NY2, nwj, ng; // QP: row pitch of the Y fields
     size_t YS;
     int mfma;                   // use the matrix-core kernels when the tables fit
     int has_mid, rows_m, njp, KL; // matrix-core shape (set by their launchers)
@@ -38,7 +38,7 @@ struct DctArgs {
     const double *wavx, *wavz;
     double Re;
     zd *bcw;           // curl: the curl part of the pressure wall condition [q][2], or null
-    int ny, JS, NQ, nzk, NY2, L, nf, curl, CH;
+    int ny, JS, NQ, QP, nzk, NY2, L, nf, curl, CH;
     int out32;         // forward: spec_out holds single-precision complex planes
 };
 bool dct_supported(int L);
@@ -52,7 +52,7 @@ struct ZArgs {
     size_t in_fs, out_fs; // field strides, complex elements
     const void *tw;
     FftPlan plan;
-    int nkx, nzk, NZS, NQ, KT, NL;
+    int nkx, nzk, NZS, QP, KT, NL;
     int rf; // use the register-resident FFT when available
     int nkxg; // register z forward: kx groups per (field, l)
     int pair; // FFT rows on lane pairs (even factors)

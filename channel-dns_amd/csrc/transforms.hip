@@ -82,9 +82,9 @@ __global__ void __launch_bounds__(512) k_ybwd(YArgs a) {
     for (int k = 0; k < LW; ++k) {
         const int lp = l0 + k;
         if (lp < NLH) {
-            out[(size_t)lp * a.NQ + q] = accE[k] + accO[k];
+            out[(size_t)lp * a.QP + q] = accE[k] + accO[k];
             const int lm = a.NY2 - lp;
-            if (lm != lp) out[(size_t)lm * a.NQ + q] = accE[k] - accO[k];
+            if (lm != lp) out[(size_t)lm * a.QP + q] = accE[k] - accO[k];
         }
     }
 }
@@ -114,10 +114,10 @@ __global__ void __launch_bounds__(512) k_yfwd(YArgs a) {
             const int lp = l0 + lc, q = q0 + ql;
             cpx<R> s = {R(0), R(0)}, d = {R(0), R(0)};
             if (lp < NLH && q < a.NQ) {
-                const cpx<R> y1 = Y[(size_t)lp * a.NQ + q];
+                const cpx<R> y1 = Y[(size_t)lp * a.QP + q];
                 const int lm = NY2 - lp;
                 if (lm != lp) {
-                    const cpx<R> y2 = Y[(size_t)lm * a.NQ + q];
+                    const cpx<R> y2 = Y[(size_t)lm * a.QP + q];
                     s = y1 + y2;
                     d = y1 - y2;
                 } else {
@@ -176,7 +176,7 @@ __global__ void __launch_bounds__(256) k_zbwd(ZArgs a) {
     const int kt0 = blockIdx.x * a.KT, l = blockIdx.y, f = blockIdx.z;
     const int nl = min(a.KT, a.nkx - kt0);
     const int N = a.plan.n, NZS = a.NZS;
-    const cpx<R> *__restrict__ Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.NQ;
+    const cpx<R> *__restrict__ Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.QP;
     for (int e = threadIdx.x; e < nl * N; e += blockDim.x) {
         const int ln = e / N, s = e - ln * N;
         const int kx = kt0 + ln;
@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(256) k_zfwd(ZArgs a) {
     __syncthreads();
     fft_block<R, IT>(buf, nl, a.plan, reinterpret_cast<const cpx<R> *>(a.tw), -1);
     const R inv = R(1.0 / N);
-    cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.NQ;
+    cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.QP;
     for (int e = threadIdx.x; e < nl * a.nzk; e += blockDim.x) {
         const int ln = e / a.nzk, kzi = e - ln * a.nzk;
         const int kz = kzi - NZS;

@@ -182,7 +182,7 @@ __global__ void __launch_bounds__((64 * Dct2Geo<R, N1, N2>::W)) k_ybwd_dct2(DctA
     cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.y) + (size_t)f * a.YS + q0;
     for (int e = threadIdx.x; e < NL * QB; e += blockDim.x) {
         const int l = e / QB, c = e - l * QB;
-        if (c < nq) Y[(size_t)l * a.NQ + c] = buf[e];
+        if (c < nq) Y[(size_t)l * a.QP + c] = buf[e];
     }
 }
 
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__((64 * Dct2Geo<R, N1, N2>::W)) k_yfwd_dct2(DctA
         const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.y) + (size_t)f * a.YS + q0;
         for (int e = threadIdx.x; e < NL * QB; e += blockDim.x) {
             const int l = e / QB, c = e - l * QB;
-            buf[e] = c < nq ? Y[(size_t)l * a.NQ + c] : cpx<R>{R(0), R(0)};
+            buf[e] = c < nq ? Y[(size_t)l * a.QP + c] : cpx<R>{R(0), R(0)};
         }
     }
     __syncthreads();

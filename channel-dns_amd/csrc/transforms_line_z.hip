@@ -17,7 +17,7 @@ __global__ void __launch_bounds__(512) k_zbwd_line(ZArgs a, LinePlan p) {
     const int lf = L / nb, kx0 = (L - lf * nb) * KT, f = lf / a.NL, l = lf - f * a.NL;
     const int nl = min(KT, a.nkx - kx0);
     const bool on = g < p.ng && line < nl;
-    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.NQ +
+    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.QP +
                       (size_t)(on ? kx0 + line : 0) * a.nzk;
     load_line_roots<R>(tw, a.tw, N);
     __syncthreads();
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(64) k_zfwd_line(ZArgs a, LinePlan p) {
     pass_a<R, -1, BIG>(p, t, on, tw, T, [&](int n) { return Z[n]; }, NoSync{});
     lsync();
     const R inv = R(1.0 / N);
-    cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.NQ + (size_t)(on ? kx : 0) * a.nzk;
+    cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.QP + (size_t)(on ? kx : 0) * a.nzk;
     pass_b<R, -1, BIG>(
         p, t, on, T,
         [&](int s, cpx<R> v) {

@@ -373,7 +373,7 @@ __global__ void __launch_bounds__((kZThreads<R, N1, N2>)) k_zbwd_rf(ZArgs a) {
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
-    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.NQ +
+    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.QP +
                       (size_t)(valid ? kx : 0) * a.nzk;
     cpx<R> x[MX];
     sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
@@ -423,7 +423,7 @@ __global__ void __launch_bounds__(64) k_zfwd_rf(ZArgs a) {
     two_pass<R, N1, N2, -1>(x, t, tw, buf[g], lsync);
     if (valid && t < N2) {
         const R inv = R(1.0 / N);
-        cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.NQ + (size_t)kx * a.nzk;
+        cpx<R> *Y = reinterpret_cast<cpx<R> *>(a.out) + (size_t)f * a.out_fs + (size_t)l * a.QP + (size_t)kx * a.nzk;
         sfor<0, N1>([&](auto k1) {
             const int s = t + N2 * decltype(k1)::value;
             // when N = 2 NZS the slot NZS serves both kz = NZS and kz = -NZS, halved on the
@@ -467,7 +467,7 @@ __global__ void __launch_bounds__((kZPThreads<R, N1, N2>)) k_zbwd_pair(ZArgs a) 
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
-    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.NQ +
+    const cpx<R> *Y = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)f * a.in_fs + (size_t)l * a.QP +
                       (size_t)(valid ? kx : 0) * a.nzk;
     cpx<R> x[MH];
     sfor<0, MH>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });

@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(64 * W) k_ybwd_mfma(YArgs a) {
             R v = mid[c];
             v += __shfl_xor(v, 16);
             v += __shfl_xor(v, 32);
-            if (k == 0 && okq[c]) Y[((size_t)(NLH - 1) * a.NQ + q) * 2 + (col & 1)] = v;
+            if (k == 0 && okq[c]) Y[((size_t)(NLH - 1) * a.QP + q) * 2 + (col & 1)] = v;
         }
         if (!okq[c]) continue;
 #pragma unroll
@@ -232,8 +232,8 @@ __global__ void __launch_bounds__(64 * W) k_ybwd_mfma(YArgs a) {
                 const int lp = l0 + 16 * t + M::row(k, r);
                 if (lp < rows) {
                     const R e = accE[c][t][r], o = accO[c][t][r];
-                    Y[((size_t)lp * a.NQ + q) * 2 + (col & 1)] = e + o;
-                    Y[((size_t)(NY2 - lp) * a.NQ + q) * 2 + (col & 1)] = e - o;
+                    Y[((size_t)lp * a.QP + q) * 2 + (col & 1)] = e + o;
+                    Y[((size_t)(NY2 - lp) * a.QP + q) * 2 + (col & 1)] = e - o;
                 }
             }
     }
@@ -481,7 +481,7 @@ __global__ void __launch_bounds__(64 * W) k_ybwd_curl(YArgs a) {
         const R su = pair_swap(m[0]), sv = pair_swap(m[1]), sw = pair_swap(m[2]);
         const R out[6] = {m[0], m[1], m[2], m[4] - sg * kz * sv, sg * (kz * su - kx * sw), sg * kx * sv - m[3]};
         if (k == 0 && okq) {
-            const size_t o = ((size_t)(NLH - 1) * a.NQ + q) * 2 + hh;
+            const size_t o = ((size_t)(NLH - 1) * a.QP + q) * 2 + hh;
 #pragma unroll
             for (int f = 0; f < 6; ++f) Y[f * FS + o] = out[f];
         }
@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(64 * W) k_ybwd_curl(YArgs a) {
                 sm[f] = pair_swap(um[f]);
             }
             if (okq && lp < rows) {
-                const size_t op = ((size_t)lp * a.NQ + q) * 2 + hh, om = ((size_t)(NY2 - lp) * a.NQ + q) * 2 + hh;
+                const size_t op = ((size_t)lp * a.QP + q) * 2 + hh, om = ((size_t)(NY2 - lp) * a.QP + q) * 2 + hh;
 #pragma unroll
                 for (int f = 0; f < 3; ++f) {
                     Y[f * FS + op] = up[f];
@@ -585,7 +585,7 @@ __global__ void __launch_bounds__(64 * W) k_yfwd_mfma(YArgs a) {
     // byte offsets within the field (a field is < 4 GB): loads are the uniform field base plus a
     // 32-bit row offset plus this lane's column offset
     const char *Yb = reinterpret_cast<const char *>(Y);
-    const unsigned rowb = (unsigned)NQ * 2u * (unsigned)sizeof(R);
+    const unsigned rowb = (unsigned)a.QP * 2u * (unsigned)sizeof(R);
     unsigned ob[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) ob[c] = ((unsigned)(oka[c] ? qa[c] : 0) * 2u + (unsigned)pa) * (unsigned)sizeof(R);
@@ -651,7 +651,7 @@ __global__ void __launch_bounds__(64 * W) k_yfwd_mfma(YArgs a) {
             if (q >= NQ) continue;
             cpx<R> ym = {R(0), R(0)};
             if (a.has_mid) {
-                const R *pm = Y + ((size_t)(NLH - 1) * NQ + q) * 2;
+                const R *pm = Y + ((size_t)(NLH - 1) * a.QP + q) * 2;
                 ym = {pm[0], pm[1]};
             }
             zd *out = a.spec_out[f] + (size_t)q * a.JS;
