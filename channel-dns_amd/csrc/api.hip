@@ -184,6 +184,16 @@ struct cdns_ctx {
     zd *body[3] = {};
     bool body_on = false;
 
+    // the launches of kGraphSteps steady steps as a graph, one for each of the two states of the swapped
+    // planes, with what they were captured from (replay_steps)
+    struct StepGraph {
+        hipGraphExec_t exec = nullptr;
+        const void *u = nullptr, *nl = nullptr, *z = nullptr;
+        bool body = false;
+    } graph[2];
+    bool graphs = true; // false once a capture has failed
+    long steady = 0;    // steady steps of cdns_run so far
+
     // adjoint workspaces (allocated on first use; FP64 only)
     bool adj_ready = false;
     zd *a_lu[3] = {}, *a_lup[3] = {}, *a_lnp[3] = {}, *a_lbp = nullptr, *a_lf[3] = {};
@@ -852,6 +862,88 @@ void step(cdns_ctx *c, int it, bool pressure = true) {
     }
 }
 
+// A step of a small grid is six launches of a few microseconds each, and the host needs as long to issue them
+// as the device to run them (32 x 33 x 32, steps of six contexts in turn, on a host of 3.7 us a launch: 23 us a
+// step, 17 as graphs; at 72 x 73 x 72 the device needs 30 us and graphs change nothing).  So the launches of
+// kGraphSteps steady steps are captured once per context and replayed: they depend on the context's
+// buffers and coefficients only, which the steps leave as they were after an even number of swaps.
+// Capturing costs some 0.2 ms, so a context does it only after kGraphAfter steady steps.
+constexpr int kGraphSteps = 6;
+constexpr long kGraphAfter = 40, kGraphPoints = 1 << 18;
+
+// The graph of the context's current buffers; null when there is none and none could be made.
+hipGraphExec_t step_graph(cdns_ctx *c, int it) {
+    auto &s = c->graph[std::less<const void *>()(c->u[0], c->up[0])];
+    if (s.exec && s.u == c->u[0] && s.nl == c->nl[0] && s.z == c->Zbuf && s.body == c->body_on) return s.exec;
+    if (c->steady < kGraphAfter) return nullptr;
+    // another stream's capture, in this thread or another, forbids some of what follows unless relaxed
+    struct Relaxed {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+        ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    } relaxed;
+    if (s.exec) {
+        CDNS_HIP(hipStreamSynchronize(c->st)); // it may still be running
+        CDNS_HIP(hipGraphExecDestroy(s.exec));
+        s.exec = nullptr;
+    }
+    const double time = c->time;
+    zd *planes[12];
+    for (int k = 0; k < 3; ++k) {
+        planes[k] = c->u[k];
+        planes[3 + k] = c->up[k];
+        planes[6 + k] = c->nl[k];
+        planes[9 + k] = c->nlp[k];
+    }
+    hipGraph_t g = nullptr;
+    bool ok = hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal) == hipSuccess;
+    if (ok) {
+        try {
+            for (int k = 0; k < kGraphSteps; ++k) step(c, it + k, false);
+        } catch (const std::exception &) {
+            ok = false;
+        }
+        ok = hipStreamEndCapture(c->st, &g) == hipSuccess && ok;
+        ok = ok && hipGraphInstantiate(&s.exec, g, nullptr, nullptr, 0) == hipSuccess;
+        if (g) (void)hipGraphDestroy(g);
+    }
+    c->time = time;
+    for (int k = 0; k < 3; ++k) {
+        c->u[k] = planes[k];
+        c->up[k] = planes[3 + k];
+        c->nl[k] = planes[6 + k];
+        c->nlp[k] = planes[9 + k];
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        s.exec = nullptr;
+        c->graphs = false;
+        return nullptr;
+    }
+    s.u = c->u[0];
+    s.nl = c->nl[0];
+    s.z = c->Zbuf;
+    s.body = c->body_on;
+    return s.exec;
+}
+
+// Replays kGraphSteps of the `left` steps from iteration it, another to follow, where that is worthwhile;
+// false: nothing was launched.
+bool replay_steps(cdns_ctx *c, int it, int left) {
+    const Geometry &g = c->g;
+    if (!c->graphs || c->prof || it < 3 || left <= kGraphSteps || (long)g.NX2 * g.NL * g.NZ2 > kGraphPoints) return false;
+    double co[5];
+    step_coefficients(it, c->cfg.DT, c->cfg.Re, co);
+    if (!c->setup_done || c->g_v != co[4]) return false;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone; // a caller may be capturing this stream
+    if (hipStreamIsCapturing(c->st, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return false;
+    const hipGraphExec_t e = step_graph(c, it);
+    if (!e) return false;
+    CDNS_HIP(hipGraphLaunch(e, c->st));
+    for (int k = 0; k < kGraphSteps; ++k) c->time += c->cfg.DT;
+    return true;
+}
+
 // ------------------------------------------------ discrete adjoint (new) --
 // The reference has no adjoint; this transposes the step above (FP64 contexts only).
 double g_for_iteration(const cdns_ctx *c, int it) {
@@ -1435,6 +1527,8 @@ void cdns_destroy(cdns_ctx *c) {
         (void)hipEventDestroy(e.b);
     }
     for (auto e : c->pool) (void)hipEventDestroy(e);
+    for (auto &s : c->graph)
+        if (s.exec) (void)hipGraphExecDestroy(s.exec);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->hz_ck) (void)hipFree(c->hz_ck);
     if (c->hz_seg) (void)hipFree(c->hz_seg);
@@ -1849,7 +1943,16 @@ int cdns_step(cdns_ctx *c, int it) {
 
 int cdns_run(cdns_ctx *c, int it_begin, int nsteps) {
     try {
-        for (int i = 0; i < nsteps; ++i) step(c, it_begin + i, i == nsteps - 1);
+        for (int i = 0; i < nsteps;) {
+            const int it = it_begin + i;
+            if (replay_steps(c, it, nsteps - i)) {
+                i += kGraphSteps;
+                continue;
+            }
+            step(c, it, i == nsteps - 1);
+            c->steady += it >= 3;
+            ++i;
+        }
         return 0;
     } catch (const std::exception &e) {
         return fail(c, e);
