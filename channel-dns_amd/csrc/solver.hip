@@ -298,7 +298,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE <= 
 
     // ---- per-column data of the step's corrections (influence entries, sigma denominators), read
     // before the wall divergence so that its reductions cover the latency
-    const bool compact = a.compact && mode == MODE_STEP;
+    const bool compact = a.compact && (mode == MODE_STEP || mode == MODE_BPROBLEM);
     zd idc[4] = {}, sgc[2] = {};
     if (compact && a.correct) {
         const zd *I0 = a.ID[0] + (size_t)q * 2, *I1 = a.ID[1] + (size_t)q * 2;
@@ -374,31 +374,40 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE <= 
     // the B response enters with sigma_(1 - p) for P, u, w and sigma_p for v (q = (j+1) mod 2)
     const zd sp_own = p ? sig[1] : sig[0], sp_other = p ? sig[0] : sig[1];
     zd P[NE], V[3][NE];
-    if (a.correct && a.sigma && compact) {
+    const bool real_tables = compact && a.correct && (mode == MODE_BPROBLEM || a.sigma);
+    if (real_tables) {
         // a.P null: no one reads this step's pressure, so its correction tables are not read either (their
         // two values at j = ny above excepted) and it is not written:
         // Re_tau=180 88.3 us with it, 82 without (of 329 MB the pressure is 30).
-        // P += c0 P0 + c1 P1 + s PB;  v += c0 v0 + c1 v1 + s vB;  (u, w) += i (kx, kz) (c0 f0 + c1 f1 + s fB)
+        // P += c0 P0 + c1 P1 + s PB;  v += c0 v0 + c1 v1 + s vB;  (u, w) += i (kx, kz) (c0 f0 + c1 f1 + s fB); the B
+        // problem itself is corrected without the s terms (from the eight complex tables, 137 MB at Re_tau=180, its
+        // solve took 57.4 us, 44.4 from the real ones)
+        constexpr bool kS = mode == MODE_STEP;
         double r0[NE], r1[NE], rb[NE];
+        auto combined = [&](int e, zd s) {
+            const zd v = r0[e] * c0 + r1[e] * c1;
+            if constexpr (kS) return v + rb[e] * s;
+            else return v;
+        };
         if (a.P) {
             sp::load_rcol<NE>(a.PIr[0] + toff, lane, ny, r0);
             sp::load_rcol<NE>(a.PIr[1] + toff, lane, ny, r1);
-            sp::load_rcol<NE>(a.PBr + toff, lane, ny, rb);
+            if constexpr (kS) sp::load_rcol<NE>(a.PBr + toff, lane, ny, rb);
 #pragma unroll
-            for (int e = 0; e < NE; ++e) P[e] = pc[0][e] + ((r0[e] * c0 + r1[e] * c1) + rb[e] * sp_other);
+            for (int e = 0; e < NE; ++e) P[e] = pc[0][e] + combined(e, sp_other);
             sp::store_col<NE>(a.P + off, lane, ny, P);
         }
         sp::load_rcol<NE>(a.VIv[0] + toff, lane, ny, r0);
         sp::load_rcol<NE>(a.VIv[1] + toff, lane, ny, r1);
-        sp::load_rcol<NE>(a.VBv + toff, lane, ny, rb);
+        if constexpr (kS) sp::load_rcol<NE>(a.VBv + toff, lane, ny, rb);
 #pragma unroll
-        for (int e = 0; e < NE; ++e) V[1][e] = vc[1][e] + ((r0[e] * c0 + r1[e] * c1) + rb[e] * sp_own);
+        for (int e = 0; e < NE; ++e) V[1][e] = vc[1][e] + combined(e, sp_own);
         sp::load_rcol<NE>(a.VIf[0] + toff, lane, ny, r0);
         sp::load_rcol<NE>(a.VIf[1] + toff, lane, ny, r1);
-        sp::load_rcol<NE>(a.VBf + toff, lane, ny, rb);
+        if constexpr (kS) sp::load_rcol<NE>(a.VBf + toff, lane, ny, rb);
 #pragma unroll
         for (int e = 0; e < NE; ++e) {
-            const zd phi = (r0[e] * c0 + r1[e] * c1) + rb[e] * sp_other;
+            const zd phi = combined(e, sp_other);
             V[0][e] = vc[0][e] + ikmul(kx, phi);
             V[2][e] = vc[2][e] + ikmul(kz, phi);
         }
@@ -485,7 +494,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NE <= 
     }
     if constexpr (mode == MODE_BPROBLEM)
         if (a.compact) store_compact<NE>(a.ctab_b, off, lane, ny, kx, kz, P, V);
-    if (!(a.correct && a.sigma && compact) && (mode != MODE_STEP || a.P)) sp::store_col<NE>(a.P + off, lane, ny, P);
+    if (!real_tables && (mode != MODE_STEP || a.P)) sp::store_col<NE>(a.P + off, lane, ny, P);
 #pragma unroll
     for (int k = 0; k < 3; ++k) sp::store_col<NE>(a.V[k] + off, lane, ny, V[k]);
 }
