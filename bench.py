@@ -45,8 +45,9 @@ def algorithmic_bytes(cfg, esz):
         "y_forward": 3 * Y * esz + 3 * S * zc,
         # u, u_prev, N, N_prev in; the influence/B responses as 9 real columns (P and v real,
         # u = i kx phi, w = i kz phi) and 2 real ad columns, read once for the two columns
-        # kz = -m, +m of a kx that share them (nkx (NZS + 1) distinct columns); u, P out
-        "solve_step": 12 * S * zc + 11 * nkx * (cfg["NZS"] + 1) * nj * 8 + 4 * S * zc,
+        # kz = -m, +m of a kx that share them (nkx (NZS + 1) distinct columns), those of P read and P
+        # written by a run's last step only; u out
+        "solve_step": 12 * S * zc + 8 * nkx * (cfg["NZS"] + 1) * nj * 8 + 3 * S * zc,
     }
 
 
@@ -60,12 +61,12 @@ DEFAULT_YSTAGE = "mfma"
 # SQ_INSTS_VALU of one x-product launch on this workload (FP64; rocprofv3 --pmc) and the issue
 # peak it is set against: a SIMD is 16 lanes wide, so it issues one wave64 vector instruction
 # per 4 cycles; 1024 SIMDs at 2.4 GHz.
-MEASURED_VALU = {"x_product": 42.6e6}
+MEASURED_VALU = {"x_product": 40.9e6}
 VALU_PEAK_WAVE_INSTS = 1024 * 2.4e9 / 4
 
 MEASURED_TRAFFIC = {
-    "x_product": 356.3e6,
-    "solve_step": 329.2e6,
+    "x_product": 354.8e6,
+    "solve_step": 300.4e6,
 }
 
 
