@@ -875,18 +875,19 @@ constexpr long kGraphAfter = 40, kGraphPoints = 1 << 18;
 hipGraphExec_t step_graph(cdns_ctx *c, int it) {
     auto &s = c->graph[std::less<const void *>()(c->u[0], c->up[0])];
     if (s.exec && s.u == c->u[0] && s.nl == c->nl[0] && s.z == c->Zbuf && s.body == c->body_on) return s.exec;
-    if (c->steady < kGraphAfter) return nullptr;
     // another stream's capture, in this thread or another, forbids some of what follows unless relaxed
     struct Relaxed {
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
         ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
     } relaxed;
-    if (s.exec) {
+    if (s.exec) { // of other buffers (a body force set or removed): as many launched steps before the next capture
         CDNS_HIP(hipStreamSynchronize(c->st)); // it may still be running
         CDNS_HIP(hipGraphExecDestroy(s.exec));
         s.exec = nullptr;
+        c->steady = 0;
     }
+    if (c->steady < kGraphAfter) return nullptr;
     const double time = c->time;
     zd *planes[12];
     for (int k = 0; k < 3; ++k) {
