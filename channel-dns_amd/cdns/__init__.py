@@ -102,6 +102,8 @@ def lib(path=None):
                   "cdns_adjoint_run_noalloc", "cdns_xyzfft",
                   "cdns_to_physical", "cdns_plane_moments", "cdns_diagnostics"):
             getattr(L, n).restype = i
+        L.cdns_step_graph_counts.argtypes = [vp, ctypes.POINTER(ctypes.c_longlong)]
+        L.cdns_step_graph_counts.restype = None
         _LIB = L
     return _LIB
 
@@ -307,6 +309,15 @@ class Channel:
         it_begin = self.it + 1 if it_begin is None else it_begin
         self._check(lib().cdns_run(self._h, int(it_begin), int(nsteps)))
         self.it = it_begin + nsteps - 1
+
+    def step_graphs(self):
+        """Step graphs of run() so far: {"captures", "replays", "failed"}; last_error() says why one failed."""
+        n = (ctypes.c_longlong * 3)()
+        lib().cdns_step_graph_counts(self._h, n)
+        return {"captures": n[0], "replays": n[1], "failed": bool(n[2])}
+
+    def last_error(self):
+        return lib().cdns_last_error(self._h).decode()
 
     def flow_gradients(self):
         out = np.zeros(2)

@@ -191,8 +191,9 @@ struct cdns_ctx {
         const void *u = nullptr, *nl = nullptr, *z = nullptr;
         bool body = false;
     } graph[2];
-    bool graphs = true; // false once a capture has failed
+    bool graphs = true; // false once a capture has failed (the reason is in err)
     long steady = 0;    // steady steps of cdns_run so far
+    long long ncapture = 0, nreplay = 0;
 
     // adjoint workspaces (allocated on first use; FP64 only)
     bool adj_ready = false;
@@ -897,15 +898,19 @@ hipGraphExec_t step_graph(cdns_ctx *c, int it) {
         planes[9 + k] = c->nlp[k];
     }
     hipGraph_t g = nullptr;
-    bool ok = hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal) == hipSuccess;
-    if (ok) {
+    std::string why; // the first failure
+    auto worked = [&](hipError_t e, const char *what) {
+        if (e != hipSuccess && why.empty()) why = std::string(what) + ": " + hipGetErrorString(e);
+        return e == hipSuccess;
+    };
+    if (worked(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture")) {
         try {
             for (int k = 0; k < kGraphSteps; ++k) step(c, it + k, false);
-        } catch (const std::exception &) {
-            ok = false;
+        } catch (const std::exception &e) {
+            why = e.what();
         }
-        ok = hipStreamEndCapture(c->st, &g) == hipSuccess && ok;
-        ok = ok && hipGraphInstantiate(&s.exec, g, nullptr, nullptr, 0) == hipSuccess;
+        if (worked(hipStreamEndCapture(c->st, &g), "hipStreamEndCapture") && why.empty())
+            worked(hipGraphInstantiate(&s.exec, g, nullptr, nullptr, 0), "hipGraphInstantiate");
         if (g) (void)hipGraphDestroy(g);
     }
     c->time = time;
@@ -915,12 +920,14 @@ hipGraphExec_t step_graph(cdns_ctx *c, int it) {
         c->nl[k] = planes[6 + k];
         c->nlp[k] = planes[9 + k];
     }
-    if (!ok) {
+    if (!why.empty()) { // the steps are launched one by one from here on
         (void)hipGetLastError();
         s.exec = nullptr;
         c->graphs = false;
+        c->err = "step graph: " + why;
         return nullptr;
     }
+    ++c->ncapture;
     s.u = c->u[0];
     s.nl = c->nl[0];
     s.z = c->Zbuf;
@@ -941,6 +948,7 @@ bool replay_steps(cdns_ctx *c, int it, int left) {
     const hipGraphExec_t e = step_graph(c, it);
     if (!e) return false;
     CDNS_HIP(hipGraphLaunch(e, c->st));
+    ++c->nreplay;
     for (int k = 0; k < kGraphSteps; ++k) c->time += c->cfg.DT;
     return true;
 }
@@ -1958,6 +1966,14 @@ int cdns_run(cdns_ctx *c, int it_begin, int nsteps) {
     } catch (const std::exception &e) {
         return fail(c, e);
     }
+}
+
+// For the tests and for whoever looks into a context's speed, not part of the header: captures and replays of
+// the step graphs so far, and 1 if a capture failed (cdns_last_error then holds why, until another call fails).
+void cdns_step_graph_counts(const cdns_ctx *c, long long out[3]) {
+    out[0] = c ? c->ncapture : 0;
+    out[1] = c ? c->nreplay : 0;
+    out[2] = c && !c->graphs;
 }
 
 int cdns_flow_gradients(cdns_ctx *c, double out[2]) {
