@@ -184,13 +184,12 @@ struct cdns_ctx {
     zd *body[3] = {};
     bool body_on = false;
 
-    // the launches of kGraphSteps steady steps as a graph, one for each of the two states of the swapped
-    // planes, with what they were captured from (replay_steps)
+    // the launches of kGraphSteps steady steps as a graph, without and with a body force and for each of the two
+    // states of the swapped planes, with the buffers that they were captured from (replay_steps)
     struct StepGraph {
         hipGraphExec_t exec = nullptr;
         const void *u = nullptr, *nl = nullptr, *z = nullptr;
-        bool body = false;
-    } graph[2];
+    } graph[2][2];
     bool graphs = true; // false once a capture has failed (the reason is in err)
     long steady = 0;    // steady steps of cdns_run so far
     long long ncapture = 0, nreplay = 0;
@@ -866,29 +865,27 @@ void step(cdns_ctx *c, int it, bool pressure = true) {
 // A step of a small grid is six launches of a few microseconds each, and the host needs as long to issue them
 // as the device to run them (32 x 33 x 32, steps of six contexts in turn, on a host of 3.7 us a launch: 23 us a
 // step, 17 as graphs; at 72 x 73 x 72 the device needs 30 us and graphs change nothing).  So the launches of
-// kGraphSteps steady steps are captured once per context and replayed: they depend on the context's
-// buffers and coefficients only, which the steps leave as they were after an even number of swaps.
-// Capturing costs some 0.2 ms, so a context does it only after kGraphAfter steady steps.
+// kGraphSteps steady steps are captured once per context, plane order and presence of a body force, and
+// replayed: they depend on the context's buffers and coefficients only, which the steps leave as they were after
+// an even number of swaps.  A capture costs 0.1 to 0.4 ms, so a context does it only after kGraphAfter steady
+// steps: 0.28 ms on average with six contexts in turn, which the steps have made up for after some 170 (us a
+// step over the first 60, 100, 200 and 1000, launched 17.4, 17.0, 22.9, 23.5, so 21.9, 19.6, 17.9, 16.4; one
+// context alone 39.5, 39.3, 39.2, 39.1 and 39.2, 38.6, 38.1, 37.7); making and closing a context takes 4.5 ms.
 constexpr int kGraphSteps = 6;
 constexpr long kGraphAfter = 40, kGraphPoints = 1 << 18;
 
-// The graph of the context's current buffers; null when there is none and none could be made.
+// The graph of the context's current state; null when there is none and none could be made, or when it is of
+// other buffers.
 hipGraphExec_t step_graph(cdns_ctx *c, int it) {
-    auto &s = c->graph[std::less<const void *>()(c->u[0], c->up[0])];
-    if (s.exec && s.u == c->u[0] && s.nl == c->nl[0] && s.z == c->Zbuf && s.body == c->body_on) return s.exec;
+    auto &s = c->graph[c->body_on][std::less<const void *>()(c->u[0], c->up[0])];
+    if (s.exec) return s.u == c->u[0] && s.nl == c->nl[0] && s.z == c->Zbuf ? s.exec : nullptr;
+    if (c->steady < kGraphAfter) return nullptr;
     // another stream's capture, in this thread or another, forbids some of what follows unless relaxed
     struct Relaxed {
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
         ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
     } relaxed;
-    if (s.exec) { // of other buffers (a body force set or removed): as many launched steps before the next capture
-        CDNS_HIP(hipStreamSynchronize(c->st)); // it may still be running
-        CDNS_HIP(hipGraphExecDestroy(s.exec));
-        s.exec = nullptr;
-        c->steady = 0;
-    }
-    if (c->steady < kGraphAfter) return nullptr;
     const double time = c->time;
     zd *planes[12];
     for (int k = 0; k < 3; ++k) {
@@ -931,7 +928,6 @@ hipGraphExec_t step_graph(cdns_ctx *c, int it) {
     s.u = c->u[0];
     s.nl = c->nl[0];
     s.z = c->Zbuf;
-    s.body = c->body_on;
     return s.exec;
 }
 
@@ -1536,8 +1532,9 @@ void cdns_destroy(cdns_ctx *c) {
         (void)hipEventDestroy(e.b);
     }
     for (auto e : c->pool) (void)hipEventDestroy(e);
-    for (auto &s : c->graph)
-        if (s.exec) (void)hipGraphExecDestroy(s.exec);
+    for (auto &of_body : c->graph)
+        for (auto &s : of_body)
+            if (s.exec) (void)hipGraphExecDestroy(s.exec);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->hz_ck) (void)hipFree(c->hz_ck);
     if (c->hz_seg) (void)hipFree(c->hz_seg);

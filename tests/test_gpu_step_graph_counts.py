@@ -52,3 +52,18 @@ def test_timed_steps_and_first_steps_are_launched(gpu):
     for _ in range(20):
         ch.step()
     assert counts(ch) == (1, 16)
+
+
+def test_a_body_force_set_and_removed_again_has_its_own_graphs(gpu):
+    """Each state is captured once, however often the force comes and goes."""
+    ch = small(gpu)
+    force = 0.01 * fields.seeded_velocity(ch.cfg, seed=7, mean="laminar", kmax=4, amplitude=1.0)
+    ch.run(AFTER)
+    seen = []
+    for k in range(4):
+        for f in (None, force):
+            ch.set_body_force(f)
+            ch.run(20)
+            seen.append(counts(ch))
+    assert [c for c, _ in seen] == [1] + [2] * 7
+    assert [r for _, r in seen] == [3 * (k + 1) for k in range(8)]
