@@ -98,6 +98,7 @@ struct XArgs {
     int nprod;
 };
 
+int device_cus(); // compute units of the device
 void launch_ybwd(const YArgs &a, int nfields, bool fp32, hipStream_t st);
 // matrix-core variants; return false when a table does not fit the LDS budget
 bool launch_ybwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st);

@@ -48,26 +48,31 @@ __global__ void __launch_bounds__(512) k_xfwd_phys_line(XArgs a, LinePlan p) {
     const int line = wv * p.ng + g;
     const bool on = g < p.ng && 2 * line < P && p0 + 2 * line < np;
     load_line_roots<R>(tw, a.tw, N);
-    // rows wv, wv + W, ... of the block on wavefront wv, eight loads in flight
+    // rows wv, wv + W, ... of the block on wavefront wv, as many loads in flight as it has rows, up to eight
     const int W = blockDim.x >> 6, w0 = __builtin_amdgcn_readfirstlane(wv);
-    for (int j0 = w0; j0 < P; j0 += 8 * W) {
-        const double *row[8];
+    auto load_rows = [&](auto uc) {
+        constexpr int U = decltype(uc)::value;
+        for (int j0 = w0; j0 < P; j0 += U * W) {
+            const double *row[U];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int pt = min(p0 + min(j0 + u * W, P - 1), np - 1), l = pt / a.NZ2, iz = pt - l * a.NZ2;
-            row[u] = a.phys + ((size_t)iz * a.NL + l) * N;
-        }
-        for (int n = lane; n < N; n += 64) {
-            double v[8];
+            for (int u = 0; u < U; ++u) {
+                const int pt = min(p0 + min(j0 + u * W, P - 1), np - 1), l = pt / a.NZ2, iz = pt - l * a.NZ2;
+                row[u] = a.phys + ((size_t)iz * a.NL + l) * N;
+            }
+            for (int n = lane; n < N; n += 64) {
+                double v[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = row[u][n];
+                for (int u = 0; u < U; ++u) v[u] = row[u][n];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int j = j0 + u * W;
-                if (j < P) reinterpret_cast<R *>(buf + (j >> 1) * p.lb + n)[j & 1] = p0 + j < np ? R(v[u]) : R(0);
+                for (int u = 0; u < U; ++u) {
+                    const int j = j0 + u * W;
+                    if (j < P) reinterpret_cast<R *>(buf + (j >> 1) * p.lb + n)[j & 1] = p0 + j < np ? R(v[u]) : R(0);
+                }
             }
         }
-    }
+    };
+    if (W >= 4) load_rows(ic<4>{});
+    else load_rows(ic<8>{});
     __syncthreads();
     cpx<R> *T = buf + line * p.lb;
     pass_a<R, -1, BIG>(p, t, on, tw, T, [&](int n) { return T[n]; }, Lsync{});
@@ -92,32 +97,46 @@ __global__ void __launch_bounds__(512) k_xfwd_phys_line(XArgs a, LinePlan p) {
 // ------------------------------------------------------------------ launch --
 namespace {
 
-// 16 points (256-byte output rows of the forward stage in FP64) on at most 8 wavefronts
-template <typename R, bool BIG> void go_xphys_line(XArgs a, const LinePlan &p, bool backward, int nf, hipStream_t st) {
-    a.P = 16;
-    const int waves = (a.P / 2 + p.ng - 1) / p.ng;
-    const size_t lds = ((size_t)a.P / 2 * p.lb + p.n) * sizeof(cpx<R>);
-    const dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P, nf), block(64 * waves);
-    if (backward) {
-        allow_lds(k_xbwd_phys_line<R, BIG>, lds);
-        hipLaunchKernelGGL((k_xbwd_phys_line<R, BIG>), grid, block, lds, st, a, p);
-    } else {
-        allow_lds(k_xfwd_phys_line<R, BIG>, lds);
-        hipLaunchKernelGGL((k_xfwd_phys_line<R, BIG>), grid, block, lds, st, a, p);
-    }
+// 16 points (256-byte output rows of the forward stage in FP64) on at least the wavefronts that their eight lines
+// need.  Short lines need one or two, which then move all 16 rows by themselves: a grid that is resident as a
+// whole with four wavefronts a block takes four.  us per launch (about 5 of them the events'), as needed / four,
+// backward and forward: 10-point lines of 38 blocks FP64 8.5 / 6.4, 8.7 / 6.4; 42 points, 160 blocks 9.2 / 7.0,
+// 9.2 / 6.9; 96 points, 294 blocks FP32 9.3 / 8.2, 9.0 / 8.1; 144 points, 657 blocks FP64 13.4 / 11.9, 13.0 / 12.2;
+// 196 points, 1213 blocks FP32 15.8 / 14.4, 16.6 / 15.4.  Beyond that (FP64 backward: 768 blocks) the smaller
+// blocks pack better: 196 points, 1213 blocks FP64 19.2 / 21.8, 19.1 / 21.1; 30 points, 3015 blocks 14.3 / 18.5,
+// 14.6 / 17.2.
+constexpr int kXPhysPoints = 16, kXPhysWaves = 4;
+
+template <typename K> void go_xphys_line(K kernel, size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
+    a.P = kXPhysPoints;
+    const int blocks = (a.NL * a.NZ2 + a.P - 1) / a.P;
+    const size_t lds = ((size_t)a.P / 2 * p.lb + p.n) * esz;
+    allow_lds(kernel, lds);
+    int waves = (a.P / 2 + p.ng - 1) / p.ng, per_cu = 0;
+    if (waves < kXPhysWaves &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * kXPhysWaves, lds) == hipSuccess &&
+        blocks * nf <= device_cus() * per_cu)
+        waves = kXPhysWaves;
+    hipLaunchKernelGGL(kernel, dim3(blocks, nf), dim3(64 * waves), lds, st, a, p);
 }
 } // namespace
 
 bool launch_xbwd_phys_line(const XArgs &a, int nf, bool fp32, hipStream_t st) {
     LinePlan p;
     if (!line_plan(a.plan.n, p)) return false;
-    line_dispatch(p, fp32, [&](auto r, auto big) { go_xphys_line<decltype(r), decltype(big)::value>(a, p, true, nf, st); });
+    line_dispatch(p, fp32, [&](auto r, auto big) {
+        using R = decltype(r);
+        go_xphys_line(k_xbwd_phys_line<R, decltype(big)::value>, sizeof(cpx<R>), a, p, nf, st);
+    });
     return true;
 }
 bool launch_xfwd_phys_line(const XArgs &a, bool fp32, hipStream_t st) {
     LinePlan p;
     if (!line_plan(a.plan.n, p)) return false;
-    line_dispatch(p, fp32, [&](auto r, auto big) { go_xphys_line<decltype(r), decltype(big)::value>(a, p, false, 1, st); });
+    line_dispatch(p, fp32, [&](auto r, auto big) {
+        using R = decltype(r);
+        go_xphys_line(k_xfwd_phys_line<R, decltype(big)::value>, sizeof(cpx<R>), a, p, 1, st);
+    });
     return true;
 }
 

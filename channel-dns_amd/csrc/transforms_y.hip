@@ -711,7 +711,7 @@ static int tiles_per_part(size_t bytes_per_tile, size_t fixed, int cap) {
 
 // compute units of the device current at the first call (256 if the query fails); the static's
 // initialisation runs once, also when several host threads launch
-static int device_cus() {
+int device_cus() {
     static const int cus = [] {
         int dev = 0, n = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
