@@ -113,11 +113,16 @@ void launch_xfwd_phys(const XArgs &a, bool fp32, hipStream_t st);
 // register-resident two-pass FFT variants; return false for lengths without an instantiation
 bool rf_supported(int n);
 bool launch_xprod_rf(const XArgs &a, bool fp32, hipStream_t st);
+bool launch_xbwd_phys_rf(const XArgs &a, int nf, bool fp32, hipStream_t st);
+bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_zbwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 bool launch_zfwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 // two-pass FFTs of runtime factors; return false for lengths without a factor pair of the list
 bool launch_xprod_line(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_xbwd_phys_line(const XArgs &a, int nf, bool fp32, hipStream_t st);
+constexpr int kXPhysPoints = 16; // points per block of these two
+// their blocks that are resident at once: with four wavefronts each (wide), or with as many as their lines need
+int xphys_line_resident(int n, bool fp32, bool backward, bool wide);
 bool launch_xfwd_phys_line(const XArgs &a, bool fp32, hipStream_t st);
 bool launch_zbwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);
 bool launch_zfwd_line(const ZArgs &a, int nf, bool fp32, hipStream_t st);

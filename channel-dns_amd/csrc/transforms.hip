@@ -487,7 +487,7 @@ void launch_xprod(const XArgs &a, bool fp32, hipStream_t st) {
     }
 }
 void launch_xbwd_phys(const XArgs &a, int nfields, bool fp32, hipStream_t st) {
-    if (a.rf && launch_xbwd_phys_line(a, nfields, fp32, st)) return;
+    if (a.rf && (launch_xbwd_phys_rf(a, nfields, fp32, st) || launch_xbwd_phys_line(a, nfields, fp32, st))) return;
     if (nfields > 1) { // the Stockham kernel takes one field
         for (int f = 0; f < nfields; ++f) {
             XArgs b = a;
@@ -506,7 +506,7 @@ void launch_xbwd_phys(const XArgs &a, int nfields, bool fp32, hipStream_t st) {
     }
 }
 void launch_xfwd_phys(const XArgs &a, bool fp32, hipStream_t st) {
-    if (a.rf && launch_xfwd_phys_line(a, fp32, st)) return;
+    if (a.rf && (launch_xfwd_phys_rf(a, fp32, st) || launch_xfwd_phys_line(a, fp32, st))) return;
     const int it = items_per_thread(a.P / 2, a.plan);
     dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P);
     if (fp32) {

@@ -39,7 +39,8 @@ __global__ void __launch_bounds__(512) k_xbwd_phys_line(XArgs a, LinePlan p) {
     }
 }
 
-template <typename R, bool BIG>
+// U: rows in flight per wavefront (a block's 16 rows over its wavefronts)
+template <typename R, bool BIG, int U>
 __global__ void __launch_bounds__(512) k_xfwd_phys_line(XArgs a, LinePlan p) {
     extern __shared__ unsigned char smem_raw[];
     cpx<R> *tw = reinterpret_cast<cpx<R> *>(smem_raw), *buf = tw + p.n;
@@ -48,31 +49,26 @@ __global__ void __launch_bounds__(512) k_xfwd_phys_line(XArgs a, LinePlan p) {
     const int line = wv * p.ng + g;
     const bool on = g < p.ng && 2 * line < P && p0 + 2 * line < np;
     load_line_roots<R>(tw, a.tw, N);
-    // rows wv, wv + W, ... of the block on wavefront wv, as many loads in flight as it has rows, up to eight
+    // rows wv, wv + W, ... of the block on wavefront wv, U loads in flight
     const int W = blockDim.x >> 6, w0 = __builtin_amdgcn_readfirstlane(wv);
-    auto load_rows = [&](auto uc) {
-        constexpr int U = decltype(uc)::value;
-        for (int j0 = w0; j0 < P; j0 += U * W) {
-            const double *row[U];
+    for (int j0 = w0; j0 < P; j0 += U * W) {
+        const double *row[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int pt = min(p0 + min(j0 + u * W, P - 1), np - 1), l = pt / a.NZ2, iz = pt - l * a.NZ2;
+            row[u] = a.phys + ((size_t)iz * a.NL + l) * N;
+        }
+        for (int n = lane; n < N; n += 64) {
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = row[u][n];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int pt = min(p0 + min(j0 + u * W, P - 1), np - 1), l = pt / a.NZ2, iz = pt - l * a.NZ2;
-                row[u] = a.phys + ((size_t)iz * a.NL + l) * N;
-            }
-            for (int n = lane; n < N; n += 64) {
-                double v[U];
-#pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = row[u][n];
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int j = j0 + u * W;
-                    if (j < P) reinterpret_cast<R *>(buf + (j >> 1) * p.lb + n)[j & 1] = p0 + j < np ? R(v[u]) : R(0);
-                }
+                const int j = j0 + u * W;
+                if (j < P) reinterpret_cast<R *>(buf + (j >> 1) * p.lb + n)[j & 1] = p0 + j < np ? R(v[u]) : R(0);
             }
         }
-    };
-    if (W >= 4) load_rows(ic<4>{});
-    else load_rows(ic<8>{});
+    }
     __syncthreads();
     cpx<R> *T = buf + line * p.lb;
     pass_a<R, -1, BIG>(p, t, on, tw, T, [&](int n) { return T[n]; }, Lsync{});
@@ -99,34 +95,55 @@ namespace {
 
 // 16 points (256-byte output rows of the forward stage in FP64) on at least the wavefronts that their eight lines
 // need.  Short lines need one or two, which then move all 16 rows by themselves: a grid that is resident as a
-// whole with four wavefronts a block takes four.  us per launch (about 5 of them the events'), as needed / four,
+// whole with four wavefronts a block (or two) takes four (two).  us per launch (about 5 of them the events'), as needed / four,
 // backward and forward: 10-point lines of 38 blocks FP64 8.5 / 6.4, 8.7 / 6.4; 42 points, 160 blocks 9.2 / 7.0,
 // 9.2 / 6.9; 96 points, 294 blocks FP32 9.3 / 8.2, 9.0 / 8.1; 144 points, 657 blocks FP64 13.4 / 11.9, 13.0 / 12.2;
 // 196 points, 1213 blocks FP32 15.8 / 14.4, 16.6 / 15.4.  Beyond that (FP64 backward: 768 blocks) the smaller
 // blocks pack better: 196 points, 1213 blocks FP64 19.2 / 21.8, 19.1 / 21.1; 30 points, 3015 blocks 14.3 / 18.5,
 // 14.6 / 17.2.
-constexpr int kXPhysPoints = 16, kXPhysWaves = 4;
-
-template <typename K> void go_xphys_line(K kernel, size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
+constexpr int kXPhysWaves = 4;
+size_t xphys_lds(const LinePlan &p, size_t esz) { return ((size_t)kXPhysPoints / 2 * p.lb + p.n) * esz; }
+int xphys_waves(const LinePlan &p) { return (kXPhysPoints / 2 + p.ng - 1) / p.ng; }
+template <typename K> int xphys_resident(K kernel, int waves, size_t lds) {
+    int per_cu = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds) == hipSuccess ? device_cus() * per_cu : 0;
+}
+// wide: the kernel for four wavefronts a block, narrow: for fewer
+template <typename K> void go_xphys_line(K narrow, K wide, size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
     a.P = kXPhysPoints;
     const int blocks = (a.NL * a.NZ2 + a.P - 1) / a.P;
-    const size_t lds = ((size_t)a.P / 2 * p.lb + p.n) * esz;
+    const size_t lds = xphys_lds(p, esz);
+    int waves = xphys_waves(p);
+    for (int w = kXPhysWaves; w > waves; w /= 2)
+        if (blocks * nf <= xphys_resident(w < kXPhysWaves ? narrow : wide, w, lds)) waves = w;
+    const K kernel = waves < kXPhysWaves ? narrow : wide;
     allow_lds(kernel, lds);
-    int waves = (a.P / 2 + p.ng - 1) / p.ng, per_cu = 0;
-    if (waves < kXPhysWaves &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * kXPhysWaves, lds) == hipSuccess &&
-        blocks * nf <= device_cus() * per_cu)
-        waves = kXPhysWaves;
     hipLaunchKernelGGL(kernel, dim3(blocks, nf), dim3(64 * waves), lds, st, a, p);
 }
 } // namespace
+
+int xphys_line_resident(int n, bool fp32, bool backward, bool wide) {
+    LinePlan p;
+    if (!line_plan(n, p)) return 0;
+    int blocks = 0;
+    line_dispatch(p, fp32, [&](auto r, auto big) {
+        using R = decltype(r);
+        constexpr bool B = decltype(big)::value;
+        const int waves = wide ? std::max(kXPhysWaves, xphys_waves(p)) : xphys_waves(p);
+        const size_t lds = xphys_lds(p, sizeof(cpx<R>));
+        blocks = xphys_resident(backward ? k_xbwd_phys_line<R, B> : (waves < kXPhysWaves ? k_xfwd_phys_line<R, B, 8> : k_xfwd_phys_line<R, B, 4>),
+                                waves, lds);
+    });
+    return blocks;
+}
 
 bool launch_xbwd_phys_line(const XArgs &a, int nf, bool fp32, hipStream_t st) {
     LinePlan p;
     if (!line_plan(a.plan.n, p)) return false;
     line_dispatch(p, fp32, [&](auto r, auto big) {
         using R = decltype(r);
-        go_xphys_line(k_xbwd_phys_line<R, decltype(big)::value>, sizeof(cpx<R>), a, p, nf, st);
+        constexpr bool B = decltype(big)::value;
+        go_xphys_line(k_xbwd_phys_line<R, B>, k_xbwd_phys_line<R, B>, sizeof(cpx<R>), a, p, nf, st);
     });
     return true;
 }
@@ -135,7 +152,8 @@ bool launch_xfwd_phys_line(const XArgs &a, bool fp32, hipStream_t st) {
     if (!line_plan(a.plan.n, p)) return false;
     line_dispatch(p, fp32, [&](auto r, auto big) {
         using R = decltype(r);
-        go_xphys_line(k_xfwd_phys_line<R, decltype(big)::value>, sizeof(cpx<R>), a, p, 1, st);
+        constexpr bool B = decltype(big)::value;
+        go_xphys_line(k_xfwd_phys_line<R, B, 8>, k_xfwd_phys_line<R, B, 4>, sizeof(cpx<R>), a, p, 1, st);
     });
     return true;
 }

@@ -311,6 +311,93 @@ __global__ void __launch_bounds__(64 * kXWaves<R>) k_xprod_pair(XArgs a) {
     }
 }
 
+// ------------------------------------------- single-field x stages (physical) --
+// Two points share one complex line: a + i b.  Field blockIdx.y.
+template <typename R, int N1, int N2>
+__global__ void __launch_bounds__(64) k_xbwd_phys_rf(XArgs a) {
+    using Gm = Geo<N1, N2>;
+    constexpr int N = Gm::N, MX = Gm::MX, G = Gm::G, NG = Gm::NG, LB = Gm::LB;
+    __shared__ cpx<R> tw[N];
+    __shared__ cpx<R> buf[NG][LB];
+    const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
+    load_roots<R, N>(tw, a.tw);
+    __syncthreads();
+    const int np = a.NL * a.NZ2, K = a.nkx - 1;
+    const int pa = 2 * (blockIdx.x * NG + g), pb = pa + 1;
+    const cpx<R> *Z = reinterpret_cast<const cpx<R> *>(a.in) + (size_t)blockIdx.y * a.in_fs;
+    double *phys = a.phys + (size_t)blockIdx.y * a.phys_fs;
+    cpx<R> x[MX];
+    sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
+    if (t < N1 && pa < np) {
+        const cpx<R> *A = Z + (size_t)pa * a.nkx;
+        const cpx<R> *Bv = pb < np ? Z + (size_t)pb * a.nkx : nullptr;
+        sfor<0, N2>([&](auto n2) {
+            const int k = t + N1 * decltype(n2)::value;
+            x[n2] = herm_pack(A, Bv, k, N, K);
+            // coarse grid, NXS = N/2: the Nyquist coefficient doubled (transforms.cpp:576-578)
+            if (a.coarse && 2 * k == N) x[n2] = {R(2) * x[n2].x, R(2) * x[n2].y};
+        });
+    }
+    two_pass<R, N1, N2, +1>(x, t, tw, buf[g], wsync);
+    if (t < N2) {
+        sfor<0, N1>([&](auto k1) {
+            const int n = t + N2 * decltype(k1)::value;
+            if (pa < np) {
+                const int l = pa / a.NZ2, iz = pa - l * a.NZ2;
+                phys[((size_t)iz * a.NL + l) * N + n] = double(x[k1].x);
+            }
+            if (pb < np) {
+                const int l = pb / a.NZ2, iz = pb - l * a.NZ2;
+                phys[((size_t)iz * a.NL + l) * N + n] = double(x[k1].y);
+            }
+        });
+    }
+}
+
+template <typename R, int N1, int N2>
+__global__ void __launch_bounds__(64) k_xfwd_phys_rf(XArgs a) {
+    using Gm = Geo<N1, N2>;
+    constexpr int N = Gm::N, MX = Gm::MX, G = Gm::G, NG = Gm::NG, LB = Gm::LB;
+    __shared__ cpx<R> tw[N];
+    __shared__ cpx<R> buf[NG][LB];
+    const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
+    load_roots<R, N>(tw, a.tw);
+    __syncthreads();
+    const int np = a.NL * a.NZ2, K = a.nkx - 1;
+    const int pa = 2 * (blockIdx.x * NG + g), pb = pa + 1;
+    cpx<R> x[MX];
+    sfor<0, MX>([&](auto j) { x[j] = cpx<R>{R(0), R(0)}; });
+    if (t < N2) {
+        sfor<0, N1>([&](auto j) {
+            const int n = t + N2 * decltype(j)::value;
+            R re = R(0), im = R(0);
+            if (pa < np) {
+                const int l = pa / a.NZ2, iz = pa - l * a.NZ2;
+                re = R(a.phys[((size_t)iz * a.NL + l) * N + n]);
+            }
+            if (pb < np) {
+                const int l = pb / a.NZ2, iz = pb - l * a.NZ2;
+                im = R(a.phys[((size_t)iz * a.NL + l) * N + n]);
+            }
+            x[j] = {re, im};
+        });
+    }
+    two_pass<R, N2, N1, -1>(x, t, tw, buf[g], wsync);
+    cpx<R> *B = buf[g];
+    if (t < N1) sfor<0, N2>([&](auto k1) { B[t + N1 * decltype(k1)::value] = x[k1]; });
+    wsync();
+    const R half = R(0.5) / R(N);
+    cpx<R> *ZN = reinterpret_cast<cpx<R> *>(a.out);
+    for (int k = t; k <= K; k += G) {
+        const cpx<R> f = B[k], gm = conjc(B[k == 0 ? 0 : N - k]);
+        const cpx<R> s = f + gm, d = f - gm;
+        // coarse grid, NXS = N/2: the Nyquist coefficient halved (transforms.cpp:496-497)
+        const R hk = (a.coarse && 2 * k == N) ? R(0.5) * half : half;
+        if (pa < np) ZN[zline_index(pa, k, a.nkx, a.NZ2)] = {hk * s.x, hk * s.y};
+        if (pb < np) ZN[zline_index(pb, k, a.nkx, a.NZ2)] = {hk * d.y, -hk * d.x};
+    }
+}
+
 // ------------------------------------------------------------------ z stages --
 // Backward: a block owns KB (16, or 8 for the largest lengths) consecutive kx lines of one
 // (field, l), one lane group per line; its output (Z[l][iz][kx], kx contiguous) goes through an LDS
@@ -513,6 +600,25 @@ template <typename R, int N1, int N2> static void go_xprod(const XArgs &a, hipSt
     hipLaunchKernelGGL((k_xprod_rf<R, N1, N2>), dim3((a.NL * a.NZ2 + Gm::NG - 1) / Gm::NG, a.nprod), dim3(64), 0,
                        st, a);
 }
+template <typename R, int N1, int N2> static dim3 xphys_grid(const XArgs &a, int nf) {
+    constexpr int PB = 2 * Geo<N1, N2>::NG;
+    return dim3((a.NL * a.NZ2 + PB - 1) / PB, nf);
+}
+template <typename R, int N1, int N2> static void go_xbwd(const XArgs &a, int nf, hipStream_t st) {
+    const dim3 grid = xphys_grid<R, N1, N2>(a, nf);
+    hipLaunchKernelGGL((k_xbwd_phys_rf<R, N1, N2>), grid, dim3(64), 0, st, a);
+}
+// only_round: not where this grid needs a second round of blocks
+template <typename R, int N1, int N2> static bool go_xfwd(const XArgs &a, bool only_round, hipStream_t st) {
+    const dim3 grid = xphys_grid<R, N1, N2>(a, 1);
+    int per_cu = 0;
+    if (only_round &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_xfwd_phys_rf<R, N1, N2>, 64, 0) == hipSuccess &&
+        grid.x > (unsigned)(device_cus() * per_cu))
+        return false;
+    hipLaunchKernelGGL((k_xfwd_phys_rf<R, N1, N2>), grid, dim3(64), 0, st, a);
+    return true;
+}
 template <typename R, int N1, int N2> static void go_zbwd(const ZArgs &a, int nf, hipStream_t st) {
     if constexpr (N1 % 2 == 0 && N2 % 2 == 0) {
         if (a.pair) {
@@ -551,6 +657,48 @@ bool launch_xprod_rf(const XArgs &a, bool fp32, hipStream_t st) {
     const int n = a.plan.n;
 #define X(NN, A, B) case NN: if (fp32) go_xprod<float, A, B>(a, st); else go_xprod<double, A, B>(a, st); return true;
     switch (n) { CDNS_RF_SIZES(X) X(384, 16, 24) default: return false; }
+#undef X
+}
+// Which single-field x stages run here and which on the line kernels of transforms_line_phys.hip, whose blocks of
+// 16 points move the physical rows as whole runs and then wait for each other: long lines and grids that are
+// resident as a whole (with their four wavefronts a block) gain more from the runs, the others from these blocks
+// of one wavefront without barriers.  us per launch (about 5 of them the events'), line / here, by length and
+// blocks of 16 points:
+//   backward FP64 64: 512 7.6 / 8.1, 1280 12.4 / 10.1, 4096 20.7 / 16.8; 96: 768 10.6 / 11.7, 1792 18.4 / 16.1;
+//     128: 768 12.0 / 13.0, 1792 20.8 / 18.5, 4096 34.6 / 35.0, 5160 41.6 / 46.2; 144: 1792 21.4 / 22.9
+//   backward FP32 32: 1024 7.5 / 7.1, 1792 10.7 / 7.9; 64: 1280 9.1 / 9.4, 1792 12.1 / 10.0; 96: 2560 16.1 / 16.8
+//   forward FP64 64: 512 7.9 / 7.6, 4096 21.1 / 14.3; 128: 512 10.8 / 9.9, 4096 31.4 / 25.9; 196: 2560 34.8 / 30.7;
+//     but 196: 1280 20.0 / 21.0, 256: 1024 17.9 / 21.6, where this grid needs a second round of blocks
+//   forward FP32 32: 512 6.6 / 6.6, 1024 8.4 / 6.9; 48: 768 7.5 / 7.5, 1792 11.1 / 9.5; 64: 1792 11.6 / 12.2
+#define CDNS_RF_BWD32(X) X(32, 4, 8) X(36, 6, 6) X(48, 6, 8) X(64, 8, 8)
+#define CDNS_RF_BWD64(X) CDNS_RF_BWD32(X) X(72, 8, 9) X(96, 8, 12) X(120, 10, 12) X(128, 8, 16)
+#define CDNS_RF_FWD32(X) X(32, 4, 8) X(36, 6, 6) X(48, 6, 8)
+
+static int xphys_blocks(const XArgs &a, int nf) { return (a.NL * a.NZ2 + kXPhysPoints - 1) / kXPhysPoints * nf; }
+
+bool launch_xbwd_phys_rf(const XArgs &a, int nf, bool fp32, hipStream_t st) {
+    const int n = a.plan.n, blocks = xphys_blocks(a, nf);
+    if (blocks <= xphys_line_resident(n, fp32, true, true) || (n > 96 && blocks > 8 * device_cus())) return false;
+#define X(NN, A, B) case NN: go_xbwd<R, A, B>(a, nf, st); return true;
+    if (fp32) {
+        using R = float;
+        switch (n) { CDNS_RF_BWD32(X) default: return false; }
+    }
+    using R = double;
+    switch (n) { CDNS_RF_BWD64(X) default: return false; }
+#undef X
+}
+bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st) {
+    const int n = a.plan.n, blocks = xphys_blocks(a, 1);
+    if (fp32 && blocks <= 3 * device_cus()) return false;
+    const bool line_fits = !fp32 && blocks <= xphys_line_resident(n, fp32, false, false);
+#define X(NN, A, B) case NN: return go_xfwd<R, A, B>(a, line_fits, st);
+    if (fp32) {
+        using R = float;
+        switch (n) { CDNS_RF_FWD32(X) default: return false; }
+    }
+    using R = double;
+    switch (n) { CDNS_RF_SIZES(X) default: return false; }
 #undef X
 }
 bool launch_zbwd_rf(const ZArgs &a, int nf, bool fp32, hipStream_t st) {

@@ -52,3 +52,10 @@ def test_physical_transform_of_each_length(gpu, nx2, nz2, full):
 def test_physical_transform_of_more_blocks_than_are_resident(gpu, nx2):
     """151 x 256 points: 2416 blocks."""
     check(gpu, dict(mesh(nx2, 256, 0, ny2=150)))
+
+
+# 1274 (an odd number of points), 1208, 1024 and 1280 blocks of 16 points
+@pytest.mark.parametrize("nx2,nz2,ny2", [(48, 135, 150), (72, 135, 150), (120, 128, 150), (128, 128, 150),
+                                         (256, 128, 127), (192, 128, 159)])
+def test_physical_transform_where_lengths_change_kernels(gpu, nx2, nz2, ny2):
+    check(gpu, mesh(nx2, nz2, 0, ny2=ny2))
