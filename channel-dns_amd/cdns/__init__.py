@@ -113,7 +113,7 @@ def _ptr(a):
         return None
     if isinstance(a, np.ndarray):
         assert a.flags.c_contiguous
-        return ctypes.c_void_p(a.ctypes.data)
+        return a.ctypes.data_as(ctypes.c_void_p)  # holds the array: it may be the caller's contiguous copy
     return ctypes.c_void_p(a.data_ptr())  # torch tensor
 
 
