@@ -727,18 +727,21 @@ bool launch_ybwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     const size_t esz = fp32 ? 4 : 8;
     const int TR = (a.rows_m + 15) / 16;
     if ((size_t)a.njp * 16 * esz + a.njp * esz > (size_t)kLdsBudget) return false;
-    // Two row tiles per wavefront on 8-wavefront blocks; where that grid has fewer blocks than the
-    // device CUs, one row tile on 4-wavefront blocks (four times the blocks, half the work of each).
-    // us per launch, FP64, two tiles / one tile (the three tiles per part that filled the LDS before):
-    // 196 x 193 x 196 1 field 18.6 / 22.8 (25.2), 6 fields 81.7 / 109.8 (84.1); 96 x 97 x 96 1 field
-    // 9.7 / 7.8 (11.7), 6 fields 15.5 / 15.3 (15.8); 150 x 136 x 126, 204 blocks, 1 field 11.7 / 11.4 (14.7).
+    // Two row tiles per wavefront on 8-wavefront blocks (one where the tables of two do not fit: FP64 columns beyond
+    // some 240 entries); where that grid has fewer blocks than 7/8 of the device's CUs, one row tile on 4-wavefront
+    // blocks (four times the blocks, half the work of each).  us per launch, FP64, two tiles / one tile (the
+    // three tiles per part that filled the LDS before): 196 x 193 x 196 1 field 18.6 / 22.8 (25.2), 6 fields
+    // 81.7 / 109.8 (84.1); 96 x 97 x 96 1 field 9.7 / 7.8 (11.7), 6 fields 15.5 / 15.3 (15.8); 204 blocks
+    // 11.7 / 11.4 (14.7), 232 blocks of 151 and 171 entries 15.1 / 18.1 (19.0), 16.2 / 19.7 (16.4); one tile of
+    // 255 entries on 8 / 4 wavefronts: 15.3 / 16.6, 6 fields of 136 column groups 363 / 400.
     const int ncg = (a.NQ + 8 * kWaves - 1) / (8 * kWaves), trp = tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, 2);
-    const bool small = trp == 1 || ncg * ((TR + 1) / 2) * nf < device_cus();
+    const bool small = trp == 2 && 8 * ncg * ((TR + 1) / 2) * nf < 7 * device_cus();
     if (fp32) {
         if (small) go_ybwd<float, 1, kYSmallWaves>(a, TR, nf, st);
         else go_ybwd<float, 2, kWaves>(a, (TR + 1) / 2, nf, st);
     } else {
         if (small) go_ybwd<double, 1, kYSmallWaves>(a, TR, nf, st);
+        else if (trp == 1) go_ybwd<double, 1, kWaves>(a, TR, nf, st);
         else go_ybwd<double, 2, kWaves>(a, (TR + 1) / 2, nf, st);
     }
     return true;
