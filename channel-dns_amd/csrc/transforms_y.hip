@@ -727,22 +727,38 @@ bool launch_ybwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     const size_t esz = fp32 ? 4 : 8;
     const int TR = (a.rows_m + 15) / 16;
     if ((size_t)a.njp * 16 * esz + a.njp * esz > (size_t)kLdsBudget) return false;
-    // Two row tiles per wavefront on 8-wavefront blocks (one where the tables of two do not fit: FP64 columns beyond
-    // some 240 entries); where that grid has fewer blocks than 7/8 of the device's CUs, one row tile on 4-wavefront
-    // blocks (four times the blocks, half the work of each).  us per launch, FP64, two tiles / one tile (the
-    // three tiles per part that filled the LDS before): 196 x 193 x 196 1 field 18.6 / 22.8 (25.2), 6 fields
-    // 81.7 / 109.8 (84.1); 96 x 97 x 96 1 field 9.7 / 7.8 (11.7), 6 fields 15.5 / 15.3 (15.8); 204 blocks
-    // 11.7 / 11.4 (14.7), 232 blocks of 151 and 171 entries 15.1 / 18.1 (19.0), 16.2 / 19.7 (16.4); one tile of
-    // 255 entries on 8 / 4 wavefronts: 15.3 / 16.6, 6 fields of 136 column groups 363 / 400.
-    const int ncg = (a.NQ + 8 * kWaves - 1) / (8 * kWaves), trp = tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, 2);
-    const bool small = trp == 2 && 8 * ncg * ((TR + 1) / 2) * nf < 7 * device_cus();
+    // 8-wavefront blocks with as many row tiles per wavefront as make the fewest rounds of blocks: more tiles read a
+    // column fewer times but make longer blocks, and a CU's time follows the blocks that it gets, rounded up, times
+    // a block's 5.0, 7.2 (FP64 7.7) and 8.7 (two, three, four tiles).  us per launch of 2 / 3 / 4 tiles, 6 fields of 136 column
+    // groups: FP32 7 row tiles 85.0 / 84.5 / 76.8, 9: 123.6 / 111.5 / 121.4, 10: 133.7 / 141.8 / 144.6, 12: 183.6 /
+    // 171.9 / 171.7, FP64 5: 62.0 / 63.8, 6: 82.2 / 86.0; of 58 groups FP32 5: 23.3 / 21.7 / 23.9, 8: 46.6 / 50.0 /
+    // 41.7, FP64 5: 31.4 / 30.9; 1 field of 136 groups FP32 5: 12.8 / 15.6 / 17.1, 12: 36.9 / 39.3 / 33.3, of 91
+    // groups FP64 5: 15.9 / 14.9; 6 fields at Re_tau=395 (9 row tiles, 390 groups) FP32 338 / 289.  Four tiles
+    // in FP64 fit columns of up to 126 entries only and gain nothing there; one tile is for the FP64 columns beyond
+    // some 240 entries whose tables of two do not fit.
+    // Grids of fewer two-tile blocks than 14/16 (FP64 9/16) of the CUs run one row tile on 4-wavefront blocks, four
+    // times the blocks of half the work: 1 field of 15 groups FP64 12 row tiles 18.3 / 15.7, of 58 groups 4: 11.5 /
+    // 10.3, 5: 12.0 / 12.2, of 34 groups (136, 170, 204 blocks) 7: 15.1 / 13.6, 9: 16.1 / 17.4, 12: 18.9 / 23.4; FP32 of 58 groups
+    // 6: 11.2 / 10.9, 8: 14.5 / 15.8.
+    const int kCost[5] = {0, 0, 50, fp32 ? 72 : 77, 87};
+    const int ncg = (a.NQ + 8 * kWaves - 1) / (8 * kWaves), cus = device_cus();
+    const int most = tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, fp32 ? 4 : 3);
+    auto blocks = [&](int t) { return ncg * ((TR + t - 1) / t) * nf; };
+    auto cost = [&](int t) { return (blocks(t) + cus - 1) / cus * kCost[t]; };
+    int t = std::min(most, 2);
+    for (int k = 3; k <= most; ++k)
+        if (cost(k) < cost(t)) t = k;
+    const bool small = most >= 2 && 16 * blocks(2) < (fp32 ? 14 : 9) * cus;
     if (fp32) {
         if (small) go_ybwd<float, 1, kYSmallWaves>(a, TR, nf, st);
-        else go_ybwd<float, 2, kWaves>(a, (TR + 1) / 2, nf, st);
+        else if (t == 2) go_ybwd<float, 2, kWaves>(a, (TR + 1) / 2, nf, st);
+        else if (t == 3) go_ybwd<float, 3, kWaves>(a, (TR + 2) / 3, nf, st);
+        else go_ybwd<float, 4, kWaves>(a, (TR + 3) / 4, nf, st);
     } else {
         if (small) go_ybwd<double, 1, kYSmallWaves>(a, TR, nf, st);
-        else if (trp == 1) go_ybwd<double, 1, kWaves>(a, TR, nf, st);
-        else go_ybwd<double, 2, kWaves>(a, (TR + 1) / 2, nf, st);
+        else if (t == 1) go_ybwd<double, 1, kWaves>(a, TR, nf, st);
+        else if (t == 2) go_ybwd<double, 2, kWaves>(a, (TR + 1) / 2, nf, st);
+        else go_ybwd<double, 3, kWaves>(a, (TR + 2) / 3, nf, st);
     }
     return true;
 }
