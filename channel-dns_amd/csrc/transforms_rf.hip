@@ -455,8 +455,9 @@ __global__ void __launch_bounds__((kZThreads<R, N1, N2>)) k_zbwd_rf(ZArgs a) {
     const int line = wv * NG + g;
     load_roots<R, N>(tw, a.tw);
     __syncthreads();
-    const int nb = (a.nkx + kZLines - 1) / kZLines, L = xcd_run((int)gridDim.x, kZRun * nb);
-    const int lf = L / nb, kx0 = (L - lf * nb) * kZLines, kx = kx0 + line, f = lf / a.NL, l = lf - f * a.NL;
+    int b, l, f;
+    a.order.block(a.NL, b, l, f);
+    const int kx0 = b * kZLines, kx = kx0 + line;
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
@@ -496,8 +497,8 @@ __global__ void __launch_bounds__(64) k_zfwd_rf(ZArgs a) {
     __shared__ cpx<R> buf[NG][LB];
     const int lane = threadIdx.x, g = lane / G, t = lane - g * G;
     // neighbouring kx groups of one (field, l) read the same cache lines: keep them on one XCD
-    const int L = xcd_run((int)gridDim.x, kZRun * a.nkxg);
-    const int kxg = L % a.nkxg, lf = L / a.nkxg, l = lf % a.NL, f = lf / a.NL;
+    int kxg, l, f;
+    a.order.block(a.NL, kxg, l, f);
     const int kx = kxg * NG + g;
     const bool valid = kx < a.nkx;
     const int NZS = a.NZS;
@@ -549,8 +550,9 @@ __global__ void __launch_bounds__((kZPThreads<R, N1, N2>)) k_zbwd_pair(ZArgs a) 
     __shared__ cpx<R> lds[T::LDS];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane / G, r = lane - g * G, t = r >> 1, h = r & 1;
     const int line = wv * NG + g;
-    const int nb = (a.nkx + kZLines - 1) / kZLines, L = xcd_run((int)gridDim.x, kZRun * nb);
-    const int lf = L / nb, kx0 = (L - lf * nb) * kZLines, kx = kx0 + line, f = lf / a.NL, l = lf - f * a.NL;
+    int b, l, f;
+    a.order.block(a.NL, b, l, f);
+    const int kx0 = b * kZLines, kx = kx0 + line;
     const int nl = min(kZLines, a.nkx - kx0);
     const bool valid = line < nl;
     const int NZS = a.NZS;
@@ -619,24 +621,27 @@ template <typename R, int N1, int N2> static bool go_xfwd(const XArgs &a, bool o
     hipLaunchKernelGGL((k_xfwd_phys_rf<R, N1, N2>), grid, dim3(64), 0, st, a);
     return true;
 }
+static ZArgs ordered(ZArgs a, int nb, int nf) {
+    a.order = ZOrder(nb, a.NL, nf, kZRun);
+    return a;
+}
 template <typename R, int N1, int N2> static void go_zbwd(const ZArgs &a, int nf, hipStream_t st) {
     if constexpr (N1 % 2 == 0 && N2 % 2 == 0) {
         if (a.pair) {
             using T = ZTileP<R, N1, N2>;
-            hipLaunchKernelGGL((k_zbwd_pair<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB * a.NL * nf),
-                               dim3(64 * T::WAVES), 0, st, a);
+            const int nb = (a.nkx + T::KB - 1) / T::KB;
+            hipLaunchKernelGGL((k_zbwd_pair<R, N1, N2>), dim3(nb * a.NL * nf), dim3(64 * T::WAVES), 0, st,
+                               ordered(a, nb, nf));
             return;
         }
     }
     using T = ZTile<R, N1, N2>;
-    hipLaunchKernelGGL((k_zbwd_rf<R, N1, N2>), dim3((a.nkx + T::KB - 1) / T::KB * a.NL * nf), dim3(64 * T::WAVES), 0,
-                       st, a);
+    const int nb = (a.nkx + T::KB - 1) / T::KB;
+    hipLaunchKernelGGL((k_zbwd_rf<R, N1, N2>), dim3(nb * a.NL * nf), dim3(64 * T::WAVES), 0, st, ordered(a, nb, nf));
 }
 template <typename R, int N1, int N2> static void go_zfwd(const ZArgs &a, int nf, hipStream_t st) {
-    using Gm = Geo<N1, N2>;
-    ZArgs b = a;
-    b.nkxg = (a.nkx + Gm::NG - 1) / Gm::NG;
-    hipLaunchKernelGGL((k_zfwd_rf<R, N1, N2>), dim3(b.nkxg * a.NL * nf), dim3(64), 0, st, b);
+    const int nb = (a.nkx + Geo<N1, N2>::NG - 1) / Geo<N1, N2>::NG;
+    hipLaunchKernelGGL((k_zfwd_rf<R, N1, N2>), dim3(nb * a.NL * nf), dim3(64), 0, st, ordered(a, nb, nf));
 }
 
 // Supported lengths: N = N1 * N2 with N1, N2 <= 16; the z stages also take the longer lines
