@@ -488,15 +488,8 @@ void launch_xprod(const XArgs &a, bool fp32, hipStream_t st) {
 }
 void launch_xbwd_phys(const XArgs &a, int nfields, bool fp32, hipStream_t st) {
     if (a.rf && (launch_xbwd_phys_rf(a, nfields, fp32, st) || launch_xbwd_phys_line(a, nfields, fp32, st))) return;
-    if (nfields > 1) { // the Stockham kernel takes one field
-        for (int f = 0; f < nfields; ++f) {
-            XArgs b = a;
-            b.in = static_cast<const char *>(a.in) + (size_t)f * a.in_fs * (fp32 ? sizeof(cpx<float>) : sizeof(cpx<double>));
-            b.phys = a.phys + (size_t)f * a.phys_fs;
-            launch_xbwd_phys(b, 1, fp32, st);
-        }
-        return;
-    }
+    // the Stockham kernels take one product-grid field; all coarse-grid lengths have kernels above
+    if (a.coarse || nfields > 1) throw std::logic_error("no kernel for a coarse x transform of this length");
     const int it = items_per_thread(a.P / 2, a.plan);
     dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P);
     if (fp32) {
@@ -507,6 +500,7 @@ void launch_xbwd_phys(const XArgs &a, int nfields, bool fp32, hipStream_t st) {
 }
 void launch_xfwd_phys(const XArgs &a, bool fp32, hipStream_t st) {
     if (a.rf && (launch_xfwd_phys_rf(a, fp32, st) || launch_xfwd_phys_line(a, fp32, st))) return;
+    if (a.coarse) throw std::logic_error("no kernel for a coarse x transform of this length");
     const int it = items_per_thread(a.P / 2, a.plan);
     dim3 grid((a.NL * a.NZ2 + a.P - 1) / a.P);
     if (fp32) {
