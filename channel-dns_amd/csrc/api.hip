@@ -228,7 +228,7 @@ struct cdns_ctx {
     zd *bnd_stage = nullptr; // boundary staging
     double *phys_stage = nullptr;
 
-    std::vector<void *> allocs;
+    std::vector<void *> allocs, pinned; // device and pinned host memory, given back with the context
 
     // profiling
     bool prof = false;
@@ -244,6 +244,12 @@ struct cdns_ctx {
         CDNS_HIP(hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(T)));
         CDNS_HIP(hipMemsetAsync(p, 0, std::max<size_t>(n, 1) * sizeof(T), st));
         allocs.push_back(p);
+        return static_cast<T *>(p);
+    }
+    template <typename T> T *alloc_pinned(size_t n) {
+        void *p = nullptr;
+        CDNS_HIP(hipHostMalloc(&p, std::max<size_t>(n, 1) * sizeof(T), hipHostMallocDefault));
+        pinned.push_back(p);
         return static_cast<T *>(p);
     }
     hipEvent_t ev() {
@@ -465,8 +471,8 @@ void ensure_coarse(cdns_ctx *c) {
     const size_t ns = (size_t)NLc * moment_parts(NLc);
     c->csums = c->alloc<double>(ns * kPlaneSums);
     c->cflags = c->alloc<int>(4 * kFiniteBlocks + ns);
-    CDNS_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->hsums), ns * kPlaneSums * sizeof(double), hipHostMallocDefault));
-    CDNS_HIP(hipHostMalloc(reinterpret_cast<void **>(&c->hflags), (4 * kFiniteBlocks + ns) * sizeof(int), hipHostMallocDefault));
+    c->hsums = c->alloc_pinned<double>(ns * kPlaneSums);
+    c->hflags = c->alloc_pinned<int>(4 * kFiniteBlocks + ns);
     // Clenshaw-Curtis weights on [-1, 1] over height 2 (diagnostics.cpp:17-33)
     const int n = g.NY;
     const double pi = std::acos(-1.0);
@@ -1538,8 +1544,7 @@ void cdns_destroy(cdns_ctx *c) {
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->hz_ck) (void)hipFree(c->hz_ck);
     if (c->hz_seg) (void)hipFree(c->hz_seg);
-    if (c->hsums) (void)hipHostFree(c->hsums);
-    if (c->hflags) (void)hipHostFree(c->hflags);
+    for (void *p : c->pinned) (void)hipHostFree(p);
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
 }
