@@ -254,7 +254,7 @@ def c5_adjoint(cdns, config, fields):
             S = (2 * g["NZS"] + 1) * (g["NXS"] + 1) * ((g["NYS"] + 1 + 7) // 8 * 8)
             Z = (g["NY2"] + 1) * g["NZ2"] * (g["NXS"] + 1)
             nq = (2 * g["NZS"] + 1) * (g["NXS"] + 1)
-            res["horizon_storage_bytes"] = (-(-nsteps // kc) * (9 * S + 2 * nq) + kc * 6 * Z) * 16
+            res["horizon_storage_bytes"] = ((-(-nsteps // kc) - 1) * (9 * S + 2 * nq) + kc * 6 * Z) * 16
             res["adjoint_workspace_bytes"] = free1 - free2
             res["forward_s"] = t_fwd
             res["gradient_s"] = t_adj

@@ -1203,7 +1203,7 @@ int fail(cdns_ctx *c, const std::exception &e) {
 struct HorizonSize {
     int kc = 0, nck = 0;
     size_t ckn = 0;       // complex entries per checkpoint
-    size_t ck_bytes = 0;  // all checkpoints
+    size_t ck_bytes = 0;  // all checkpoints: one per segment but the last, whose fields stay in the segment storage
     size_t seg_bytes = 0; // one segment
 };
 
@@ -1214,7 +1214,7 @@ HorizonSize horizon_size(const cdns_ctx *c, int nsteps, int k_ckpt) {
     h.kc = std::min(k_ckpt, nsteps);
     h.nck = (nsteps + h.kc - 1) / h.kc;
     h.ckn = (size_t)9 * g.S + (size_t)g.NQ * 2;
-    h.ck_bytes = (size_t)h.nck * h.ckn * sizeof(zd);
+    h.ck_bytes = (size_t)(h.nck - 1) * h.ckn * sizeof(zd);
     h.seg_bytes = (size_t)h.kc * 6 * g.ZS * c->esz;
     return h;
 }

@@ -143,13 +143,14 @@ int cdns_adjoint_step(cdns_ctx *ctx, int it, const double *velocity, double *adj
                       double *adj_velocity_prev, double *adj_nonlinear_prev,
                       double *adj_pressure_bc_prev, double *adj_force, int where);
 /* Gradient of objective(u(T)) after iterations 1..nsteps from u0 (zero history) with body force
- * `force` (or none): forward with a checkpoint every k_ckpt steps, then per segment a forward
- * recomputation that keeps each step's synthesised (u, curl u), and the adjoint steps in reverse.
+ * `force` (or none): forward with a checkpoint every k_ckpt steps and, in the last segment, each step's
+ * synthesised (u, curl u) kept; then per segment, after a forward recomputation that keeps these fields
+ * (the last segment needs none), the adjoint steps in reverse.
  * Writes J, grad_u0 and (if non-NULL) grad_force.  The context's state (velocity and history) is
  * overwritten; its time and its body force (cdns_set_body_force) are restored.  The checkpoints
  * and one segment's fields stay allocated with the context between calls (grown when a call needs
- * more): (ceil(nsteps / k_ckpt) (9 S + 2 NQ) + k_ckpt * 6 Z) * 16 bytes, S, Z and NQ the spectral,
- * z-physical and column counts. */
+ * more): ((ceil(nsteps / k_ckpt) - 1) (9 S + 2 NQ) + min(k_ckpt, nsteps) * 6 Z) * 16 bytes, S, Z and NQ the
+ * spectral, z-physical and column counts. */
 int cdns_adjoint_run(cdns_ctx *ctx, const double *u0, const double *force, int nsteps, int k_ckpt,
                      int objective, double *grad_u0, double *grad_force, double *J, int where);
 
