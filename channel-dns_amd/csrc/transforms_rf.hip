@@ -683,7 +683,10 @@ static int xphys_blocks(const XArgs &a, int nf) { return (a.NL * a.NZ2 + kXPhysP
 
 bool launch_xbwd_phys_rf(const XArgs &a, int nf, bool fp32, hipStream_t st) {
     const int n = a.plan.n, blocks = xphys_blocks(a, nf);
-    if (blocks <= xphys_line_resident(n, fp32, true, true) || (n > 96 && blocks > 8 * device_cus())) return false;
+#define X(NN, A, B) || n == NN
+    const bool here = fp32 ? false CDNS_RF_BWD32(X) : false CDNS_RF_BWD64(X);
+#undef X
+    if (!here || blocks <= xphys_line_resident(n, fp32, true, true) || (n > 96 && blocks > 8 * device_cus())) return false;
 #define X(NN, A, B) case NN: go_xbwd<R, A, B>(a, nf, st); return true;
     if (fp32) {
         using R = float;
@@ -695,7 +698,7 @@ bool launch_xbwd_phys_rf(const XArgs &a, int nf, bool fp32, hipStream_t st) {
 }
 bool launch_xfwd_phys_rf(const XArgs &a, bool fp32, hipStream_t st) {
     const int n = a.plan.n, blocks = xphys_blocks(a, 1);
-    if (fp32 && blocks <= 3 * device_cus()) return false;
+    if (!rf_supported(n) || (fp32 && blocks <= 3 * device_cus())) return false;
     const bool line_fits = !fp32 && blocks <= xphys_line_resident(n, fp32, false, false);
 #define X(NN, A, B) case NN: return go_xfwd<R, A, B>(a, line_fits, st);
     if (fp32) {
