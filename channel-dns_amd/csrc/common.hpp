@@ -51,7 +51,7 @@ struct Geometry {
     int nkx, nzk, nj, JS, NQ, NL, NLH, E;
     int QP; // row pitch of the Y fields: NQ to whole cache lines
     size_t S;  // complex entries of one spectral component plane = NQ*JS
-    size_t YS; // complex entries of one Y field = NL*NQ
+    size_t YS; // complex entries of one Y field = NL*QP
     size_t ZS; // complex entries of one Z field = NL*NZ2*nkx
 };
 

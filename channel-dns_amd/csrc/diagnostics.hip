@@ -125,7 +125,7 @@ __global__ void __launch_bounds__(256) k_plane_moments(DiagArgs a) {
     }
     if (threadIdx.x == 0) a.finite[iy * a.parts + part] = all;
 }
-// four to eight workgroups per CU over all planes, at most 16 per plane
+// at most 1024 workgroups over all planes (up to four per CU), at most 16 per plane
 int moment_parts(int NL) { return std::max(1, std::min(16, 1024 / NL)); }
 void launch_plane_moments(const DiagArgs &a, hipStream_t st) {
     hipLaunchKernelGGL(k_plane_moments, dim3(a.NL, a.parts), dim3(256), 0, st, a);

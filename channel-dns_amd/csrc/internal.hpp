@@ -106,13 +106,14 @@ __host__ __device__ inline size_t zline_index(int p, int kx, int nkx, int NZ2) {
     return ((size_t)l * nkx + kx) * NZ2 + iz;
 }
 
-// Order of the x and z stages' blocks over the XCDs (xcd_run).  Rows of nkx or NZ2 values are no whole number of
+// Order of the x and z stages' blocks over the XCDs (xcd_run, ZOrder).  Rows of nkx or NZ2 values are no whole number of
 // cache lines, and neighbouring blocks write (or read) the two parts of a line: on one XCD they meet in its L2,
 // dealt out block by block each part went to memory by itself.  Whole eighths of the grid per XCD (xcd_block)
 // also do that, but the XCDs then work far apart, which costs the x product more than it gains.  us per launch,
 // block by block / in eighths / in these runs: z backward 196 x 193 x 196 FP64 90.3 / 84.3 / 80.9, FP32
 // 51.0 / 40.2 / 40.8, 384 x 289 x 288 FP32 258 / 244 / 243; x product 106.9 / 109.0 / 105.0, 64.0 / 66.9 / 63.1,
-// 466 / 442 / 437; z forward (before in eighths) FP64 42.4 / 41.3, FP32 23.4 / 22.6, 123 / 117.  The kernels of
+// 466 / 442 / 437; z forward (before in eighths) FP64 42.4 / 41.3, FP32 23.4 / 22.6, 123 / 117 (the z stages with the divisions
+// that ZOrder took out).  The kernels of
 // runtime factors go in eighths (150 x 136 x 126 FP64: x product 61.2 / 59.5 / 62.9, z backward 35.4 / 34.3 / 35.4);
 // the x stages of physical fields, whose rows there are whole runs, block by block (41.3 / 42.3 / 43.1).
 constexpr int kXRun = 128; // points

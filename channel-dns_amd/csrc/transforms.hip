@@ -9,8 +9,8 @@
 //   x stage : c2r of (u,v,w,wx,wy,wz) packed two real lines per complex FFT, the cross
 //             product in LDS, and r2c of the three products, in one kernel, so that the
 //             nine physical fields never reach HBM.
-// The FFT kernels of this file serve the lengths that neither transforms_rf.hip (tuned) nor
-// transforms_line.hip (factor pairs up to 27) takes, e.g. 245 = 5 x 49, and CDNS_FFT=stockham.
+// The FFT kernels of this file serve the lengths that neither transforms_rf.hip (tuned) nor the line kernels
+// (linefft.hpp: factor pairs up to 27; transforms_line_x.hip, _z.hip and _phys.hip) take, e.g. 245 = 5 x 49, and CDNS_FFT=stockham.
 // Normalisation follows transforms.cpp exactly: backward synthesis is the exact value of
 // the truncated series; forward applies 1/NX2 (no Nyquist halving), 1/NZ2 and the DCT-I
 // weights 1/(2 NY2) (iy=0), 1/NY2 (iy>=1).

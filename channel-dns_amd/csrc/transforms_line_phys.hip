@@ -95,18 +95,23 @@ namespace {
 
 // 16 points (256-byte output rows of the forward stage in FP64) on at least the wavefronts that their eight lines
 // need.  Short lines need one or two, which then move all 16 rows by themselves: a grid that is resident as a
-// whole with four wavefronts a block (or two) takes four (two).  us per launch (about 5 of them the events'), as needed / four,
-// backward and forward: 10-point lines of 38 blocks FP64 8.5 / 6.4, 8.7 / 6.4; 42 points, 160 blocks 9.2 / 7.0,
-// 9.2 / 6.9; 96 points, 294 blocks FP32 9.3 / 8.2, 9.0 / 8.1; 144 points, 657 blocks FP64 13.4 / 11.9, 13.0 / 12.2;
-// 196 points, 1213 blocks FP32 15.8 / 14.4, 16.6 / 15.4.  Beyond that (FP64 backward: 768 blocks) the smaller
-// blocks pack better: 196 points, 1213 blocks FP64 19.2 / 21.8, 19.1 / 21.1; 30 points, 3015 blocks 14.3 / 18.5,
-// 14.6 / 17.2.
+// whole with four wavefronts a block (or two) takes four (two).  us per launch (about 5 of them the events'), as
+// needed / four, backward and forward: 10-point lines of 38 blocks FP64 8.5 / 6.4, 8.7 / 6.4; 42 points, 160 blocks
+// 9.2 / 7.0, 9.2 / 6.9; 96 points, 294 blocks FP32 9.3 / 8.2, 9.0 / 8.1; 144 points, 657 blocks FP64 13.4 / 11.9,
+// 13.0 / 12.2; 196 points, 1213 blocks FP32 15.8 / 14.4, 16.6 / 15.4.  Beyond that (FP64 backward: 768 blocks) the
+// smaller blocks pack better: 196 points, 1213 blocks FP64 19.2 / 21.8, 19.1 / 21.1; 30 points, 3015 blocks
+// 14.3 / 18.5, 14.6 / 17.2.
 constexpr int kXPhysWaves = 4;
 size_t xphys_lds(const LinePlan &p, size_t esz) { return ((size_t)kXPhysPoints / 2 * p.lb + p.n) * esz; }
 int xphys_waves(const LinePlan &p) { return (kXPhysPoints / 2 + p.ng - 1) / p.ng; }
 template <typename K> int xphys_resident(K kernel, int waves, size_t lds) {
     int per_cu = 0;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds) == hipSuccess ? device_cus() * per_cu : 0;
+    allow_lds(kernel, lds);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return device_cus() * per_cu;
 }
 // wide: the kernel for four wavefronts a block, narrow: for fewer
 template <typename K> void go_xphys_line(K narrow, K wide, size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
@@ -131,8 +136,8 @@ int xphys_line_resident(int n, bool fp32, bool backward, bool wide) {
         constexpr bool B = decltype(big)::value;
         const int waves = wide ? std::max(kXPhysWaves, xphys_waves(p)) : xphys_waves(p);
         const size_t lds = xphys_lds(p, sizeof(cpx<R>));
-        blocks = xphys_resident(backward ? k_xbwd_phys_line<R, B> : (waves < kXPhysWaves ? k_xfwd_phys_line<R, B, 8> : k_xfwd_phys_line<R, B, 4>),
-                                waves, lds);
+        const auto forward = waves < kXPhysWaves ? k_xfwd_phys_line<R, B, 8> : k_xfwd_phys_line<R, B, 4>;
+        blocks = xphys_resident(backward ? k_xbwd_phys_line<R, B> : forward, waves, lds);
     });
     return blocks;
 }

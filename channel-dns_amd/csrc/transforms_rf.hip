@@ -4,7 +4,7 @@
 // lanes, one FFT line per group.  The x stage keeps the six synthesised physical lines of a
 // point in registers, forms u x w there and transforms the products back, so nothing but
 // the NXS+1 retained coefficients per line touches HBM.  Sizes without an instantiation use
-// the LDS Stockham kernels of transforms.hip.
+// the line kernels of run-time factors (linefft.hpp) or the LDS Stockham kernels of transforms.hip.
 #include "internal.hpp"
 #include "regfft.hpp"
 #include <type_traits>

@@ -729,17 +729,18 @@ bool launch_ybwd_mfma(YArgs a, int nf, bool fp32, hipStream_t st) {
     if ((size_t)a.njp * 16 * esz + a.njp * esz > (size_t)kLdsBudget) return false;
     // 8-wavefront blocks with as many row tiles per wavefront as make the fewest rounds of blocks: more tiles read a
     // column fewer times but make longer blocks, and a CU's time follows the blocks that it gets, rounded up, times
-    // a block's 5.0, 7.2 (FP64 7.7) and 8.7 (two, three, four tiles).  us per launch of 2 / 3 / 4 tiles, 6 fields of 136 column
-    // groups: FP32 7 row tiles 85.0 / 84.5 / 76.8, 9: 123.6 / 111.5 / 121.4, 10: 133.7 / 141.8 / 144.6, 12: 183.6 /
-    // 171.9 / 171.7, FP64 5: 62.0 / 63.8, 6: 82.2 / 86.0; of 58 groups FP32 5: 23.3 / 21.7 / 23.9, 8: 46.6 / 50.0 /
-    // 41.7, FP64 5: 31.4 / 30.9; 1 field of 136 groups FP32 5: 12.8 / 15.6 / 17.1, 12: 36.9 / 39.3 / 33.3, of 91
-    // groups FP64 5: 15.9 / 14.9; 6 fields at Re_tau=395 (9 row tiles, 390 groups) FP32 338 / 289.  Four tiles
-    // in FP64 fit columns of up to 126 entries only and gain nothing there; one tile is for the FP64 columns beyond
-    // some 240 entries whose tables of two do not fit.
+    // a block's 5.0, 7.2 (FP64 7.7) and 8.7 (two, three, four tiles).  us per launch of 2 / 3 / 4 tiles,
+    //   6 fields of 136 column groups: FP32 7 row tiles 85.0 / 84.5 / 76.8, 9: 123.6 / 111.5 / 121.4, 10: 133.7 / 141.8 /
+    //     144.6, 12: 183.6 / 171.9 / 171.7, FP64 5: 62.0 / 63.8, 6: 82.2 / 86.0
+    //   6 fields of 58 groups: FP32 5: 23.3 / 21.7 / 23.9, 8: 46.6 / 50.0 / 41.7, FP64 5: 31.4 / 30.9
+    //   1 field: 136 groups FP32 5: 12.8 / 15.6 / 17.1, 12: 36.9 / 39.3 / 33.3, 91 groups FP64 5: 15.9 / 14.9
+    //   6 fields at Re_tau=395 (9 row tiles, 390 groups): FP32 338 / 289
+    // Four tiles in FP64 fit columns of up to 126 entries only and gain nothing there; one tile is for the FP64 columns
+    // beyond some 240 entries whose tables of two do not fit.
     // Grids of fewer two-tile blocks than 14/16 (FP64 9/16) of the CUs run one row tile on 4-wavefront blocks, four
     // times the blocks of half the work: 1 field of 15 groups FP64 12 row tiles 18.3 / 15.7, of 58 groups 4: 11.5 /
-    // 10.3, 5: 12.0 / 12.2, of 34 groups (136, 170, 204 blocks) 7: 15.1 / 13.6, 9: 16.1 / 17.4, 12: 18.9 / 23.4; FP32 of 58 groups
-    // 6: 11.2 / 10.9, 8: 14.5 / 15.8.
+    // 10.3, 5: 12.0 / 12.2, of 34 groups (136, 170, 204 blocks) 7: 15.1 / 13.6, 9: 16.1 / 17.4, 12: 18.9 / 23.4; FP32
+    // of 58 groups 6: 11.2 / 10.9, 8: 14.5 / 15.8.
     const int kCost[5] = {0, 0, 50, fp32 ? 72 : 77, 87};
     const int ncg = (a.NQ + 8 * kWaves - 1) / (8 * kWaves), cus = device_cus();
     const int most = tiles_per_part((size_t)a.njp * 16 * esz, a.njp * esz, fp32 ? 4 : 3);

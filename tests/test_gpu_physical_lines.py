@@ -59,3 +59,9 @@ def test_physical_transform_of_more_blocks_than_are_resident(gpu, nx2):
                                          (256, 128, 127), (192, 128, 159)])
 def test_physical_transform_where_lengths_change_kernels(gpu, nx2, nz2, ny2):
     check(gpu, mesh(nx2, nz2, 0, ny2=ny2))
+
+
+@pytest.mark.parametrize("nx2,ny2", [(500, 12), (625, 12), (625, 300)])
+def test_physical_transform_of_the_longest_lines(gpu, nx2, ny2):
+    """20 x 25 and 25 x 25, about the longest lengths that a context takes: a block's LDS beyond 64 KB in FP64."""
+    check(gpu, mesh(nx2, 21, 0, ny2=ny2))
