@@ -113,7 +113,9 @@ def _ptr(a):
         return None
     if isinstance(a, np.ndarray):
         assert a.flags.c_contiguous
-        return a.ctypes.data_as(ctypes.c_void_p)  # holds the array: it may be the caller's contiguous copy
+        p = ctypes.c_void_p(a.ctypes.data)
+        p.array = a  # held for the call: it may be the caller's contiguous copy
+        return p
     return ctypes.c_void_p(a.data_ptr())  # torch tensor
 
 

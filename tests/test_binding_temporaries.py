@@ -51,3 +51,22 @@ def test_copies_of_strided_arrays_outlive_the_call(monkeypatch, name):
     call, count = CALLS[name]
     call(ch, vector, scalar, boundary)
     assert [c for c in lib.calls if c[0] == name] == [(name, count, [True] * count)]
+
+
+def test_arrays_of_a_call_are_freed_with_their_last_reference(monkeypatch):
+    """Not by the cycle collector some time later: a restart's arrays are hundreds of megabytes."""
+    import gc
+
+    monkeypatch.setattr(cdns, "lib", lambda path=None: Library([]))
+    ch = object.__new__(cdns.Channel)
+    ch._h, ch.cfg, ch.nzk, ch.nj, ch.nkx = None, {}, 5, 4, 3
+    gc.disable()
+    try:
+        v = np.zeros((5, 4, 3, 3), np.complex128)
+        ch.set_state("velocity", v)
+        out = ch.get_state("velocity")
+        refs = [weakref.ref(v), weakref.ref(out)]
+        del v, out
+        assert [r() is None for r in refs] == [True, True]
+    finally:
+        gc.enable()
