@@ -104,24 +104,26 @@ namespace {
 constexpr int kXPhysWaves = 4;
 size_t xphys_lds(const LinePlan &p, size_t esz) { return ((size_t)kXPhysPoints / 2 * p.lb + p.n) * esz; }
 int xphys_waves(const LinePlan &p) { return (kXPhysPoints / 2 + p.ng - 1) / p.ng; }
-template <typename K> int xphys_resident(K kernel, int waves, size_t lds) {
-    int per_cu = 0;
-    allow_lds(kernel, lds);
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64 * waves, lds) != hipSuccess) {
+// resident blocks of `waves` wavefronts; the wavefronts that the registers of a kernel leave a CU are asked for once
+template <auto Kernel> int xphys_resident(int waves, size_t lds) {
+    static const int slots = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, Kernel, 64, 0) == hipSuccess) return n;
         (void)hipGetLastError();
         return 0;
-    }
-    return device_cus() * per_cu;
+    }();
+    constexpr size_t kCuLds = 160 * 1024;
+    return device_cus() * std::min(slots / waves, (int)(kCuLds / lds));
 }
-// wide: the kernel for four wavefronts a block, narrow: for fewer
-template <typename K> void go_xphys_line(K narrow, K wide, size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
+// Wide: the kernel for four wavefronts a block, Narrow: for fewer
+template <auto Narrow, auto Wide> void go_xphys_line(size_t esz, XArgs a, const LinePlan &p, int nf, hipStream_t st) {
     a.P = kXPhysPoints;
     const int blocks = (a.NL * a.NZ2 + a.P - 1) / a.P;
     const size_t lds = xphys_lds(p, esz);
     int waves = xphys_waves(p);
     for (int w = kXPhysWaves; w > waves; w /= 2)
-        if (blocks * nf <= xphys_resident(w < kXPhysWaves ? narrow : wide, w, lds)) waves = w;
-    const K kernel = waves < kXPhysWaves ? narrow : wide;
+        if (blocks * nf <= (w < kXPhysWaves ? xphys_resident<Narrow>(w, lds) : xphys_resident<Wide>(w, lds))) waves = w;
+    const auto kernel = waves < kXPhysWaves ? Narrow : Wide;
     allow_lds(kernel, lds);
     hipLaunchKernelGGL(kernel, dim3(blocks, nf), dim3(64 * waves), lds, st, a, p);
 }
@@ -136,8 +138,9 @@ int xphys_line_resident(int n, bool fp32, bool backward, bool wide) {
         constexpr bool B = decltype(big)::value;
         const int waves = wide ? std::max(kXPhysWaves, xphys_waves(p)) : xphys_waves(p);
         const size_t lds = xphys_lds(p, sizeof(cpx<R>));
-        const auto forward = waves < kXPhysWaves ? k_xfwd_phys_line<R, B, 8> : k_xfwd_phys_line<R, B, 4>;
-        blocks = xphys_resident(backward ? k_xbwd_phys_line<R, B> : forward, waves, lds);
+        if (backward) blocks = xphys_resident<&k_xbwd_phys_line<R, B>>(waves, lds);
+        else if (waves < kXPhysWaves) blocks = xphys_resident<&k_xfwd_phys_line<R, B, 8>>(waves, lds);
+        else blocks = xphys_resident<&k_xfwd_phys_line<R, B, 4>>(waves, lds);
     });
     return blocks;
 }
@@ -148,7 +151,7 @@ bool launch_xbwd_phys_line(const XArgs &a, int nf, bool fp32, hipStream_t st) {
     line_dispatch(p, fp32, [&](auto r, auto big) {
         using R = decltype(r);
         constexpr bool B = decltype(big)::value;
-        go_xphys_line(k_xbwd_phys_line<R, B>, k_xbwd_phys_line<R, B>, sizeof(cpx<R>), a, p, nf, st);
+        go_xphys_line<&k_xbwd_phys_line<R, B>, &k_xbwd_phys_line<R, B>>(sizeof(cpx<R>), a, p, nf, st);
     });
     return true;
 }
@@ -158,7 +161,7 @@ bool launch_xfwd_phys_line(const XArgs &a, bool fp32, hipStream_t st) {
     line_dispatch(p, fp32, [&](auto r, auto big) {
         using R = decltype(r);
         constexpr bool B = decltype(big)::value;
-        go_xphys_line(k_xfwd_phys_line<R, B, 8>, k_xfwd_phys_line<R, B, 4>, sizeof(cpx<R>), a, p, 1, st);
+        go_xphys_line<&k_xfwd_phys_line<R, B, 8>, &k_xfwd_phys_line<R, B, 4>>(sizeof(cpx<R>), a, p, 1, st);
     });
     return true;
 }

@@ -613,11 +613,15 @@ template <typename R, int N1, int N2> static void go_xbwd(const XArgs &a, int nf
 // only_round: not where this grid needs a second round of blocks
 template <typename R, int N1, int N2> static bool go_xfwd(const XArgs &a, bool only_round, hipStream_t st) {
     const dim3 grid = xphys_grid<R, N1, N2>(a, 1);
-    int per_cu = 0;
-    if (only_round &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_xfwd_phys_rf<R, N1, N2>, 64, 0) == hipSuccess &&
-        grid.x > (unsigned)(device_cus() * per_cu))
-        return false;
+    if (only_round) {
+        static const int per_cu = [] {
+            int n = 0;
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_xfwd_phys_rf<R, N1, N2>, 64, 0) == hipSuccess) return n;
+            (void)hipGetLastError();
+            return 32;
+        }();
+        if (grid.x > (unsigned)(device_cus() * per_cu)) return false;
+    }
     hipLaunchKernelGGL((k_xfwd_phys_rf<R, N1, N2>), grid, dim3(64), 0, st, a);
     return true;
 }
